@@ -20,6 +20,8 @@
 
 namespace mlau {
 
+constexpr int kMarch = 8;  // longest march of the y sweep
+
 // Single-grid kernels: the cell kernels tile their region in flattened
 // 256-cell pieces, remapped so that each XCD works on a contiguous band of
 // rows (xcd_band).
@@ -57,10 +59,11 @@ __global__ __launch_bounds__(256) void k_xsweep2d(U2 u, W2 w, G2 g)
   xsweep2d_body<ODR, FLUX, MIX>(u, w, g, W, threadIdx.x & 63);
 }
 
-template <int ODR, int FLUX, int CH, int MIX>
-__global__ __launch_bounds__(64) void k_ysweep2d(U2 u, W2 w, G2 g)
+template <int ODR, int FLUX, int MIX, bool SPLIT>
+__global__ __launch_bounds__(64) void k_ysweep2d(U2 u, W2 w, G2 g, int ch)
 {
-  ysweep2d_body<ODR, FLUX, CH, MIX>(u, w, g, blockIdx.x, blockIdx.y, threadIdx.x);
+  ysweep2d_body<ODR, FLUX, MIX, SPLIT>(u, w, g, ch, march_mid(ch, blockIdx.y, kMarch), blockIdx.x, blockIdx.y,
+                                        threadIdx.x);
 }
 
 template <int ODR>
@@ -97,10 +100,11 @@ __global__ __launch_bounds__(256) void k_xsweep2d_inl(U2 u, W2 w, G2 g)
   xsweep2d_inl_body<ODR, FLUX, MIX>(u, w, g, W, threadIdx.x & 63);
 }
 
-template <int ODR, int FLUX, int CH, int MIX, int CTW>
-__global__ __launch_bounds__(64) void k_ysweep2d_inl(U2 u, W2 w, G2 g)
+template <int ODR, int FLUX, int MIX, int CTW, bool SPLIT>
+__global__ __launch_bounds__(64) void k_ysweep2d_inl(U2 u, W2 w, G2 g, int ch)
 {
-  ysweep2d_inl_body<ODR, FLUX, CH, MIX, CTW>(u, w, g, blockIdx.x, blockIdx.y, threadIdx.x);
+  ysweep2d_inl_body<ODR, FLUX, MIX, CTW, SPLIT>(u, w, g, ch, march_mid(ch, blockIdx.y, kMarch), blockIdx.x,
+                                                blockIdx.y, threadIdx.x);
 }
 
 // CT weight 1/2 at corners 3..nx-3 x 3..ny-3 (no upwind weighting)
@@ -148,15 +152,23 @@ static void make_views(Handle *h, U2 &u0, U2 &u1, W2 &w, G2 &g)
   g.nx = h->g.nx; g.ny = h->g.ny; g.xoff = h->g.xoff; g.yoff = h->g.yoff; g.gamma = h->g.gamma;
 }
 
-template <int ODR, int FLUX, int CH, int MIX>
-static void launch_ysweep(Handle *h, const U2 &in, const W2 &w, const G2 &g)
+// Marches that may start in the middle of a longest one (march_mid).
+template <int MIX>
+static bool split_march(int ch)
 {
-  const int chunks = (g.ny - 5 + CH - 1) / CH;
-  MLAU_LAUNCH(h, K_YSWEEP2D, (k_ysweep2d<ODR, FLUX, CH, MIX>), dim3((g.nx + 63) / 64, chunks), dim3(64), in, w, g);
+  return MIX != MLAU_FP64 && ch < kMarch;
 }
 
-// Sweep launch shapes: defaults, plus the chunk lengths the tuner may pick for
-// WCNS4 with LHLLD (ODR=4; the 2048^2 vortex benchmark's scheme).
+// Faces per lane of the y sweep: march_chunk's choice, or 16, 4 or 8 with tune
+// bits 0-1 = 1, 2 or 3.
+static int ychunk(const Handle *h, const G2 &g)
+{
+  static const int fixed[4] = {0, 16, 4, 8};
+  const int t = fixed[h->tune & 3];
+  return t ? t : march_chunk((g.nx + 63) / 64, g.ny - 5, xsweep_waves(g.ny, g.nx), 0.5, kMarch,
+                              h->s.precision != MLAU_FP64);
+}
+
 template <int ODR, int FLUX, int MIX>
 static void sweeps2d(Handle *h, const U2 &in, const W2 &w, const G2 &g)
 {
@@ -165,15 +177,12 @@ static void sweeps2d(Handle *h, const U2 &in, const W2 &w, const G2 &g)
   sd.fork(1);
   MLAU_LAUNCH(h, K_XSWEEP2D, (k_xsweep2d<ODR, FLUX, MIX>), gx, dim3(256), in, w, g);
   sd.enter(0);
-  if constexpr (ODR == 4 && FLUX == FLUX_LHLLD) {  // the chunk variants for ODR=4 with LHLLD only
-    switch (h->tune & 3) {
-    case 1: launch_ysweep<ODR, FLUX, 16, MIX>(h, in, w, g); break;
-    case 2: launch_ysweep<ODR, FLUX, 4, MIX>(h, in, w, g); break;
-    default: launch_ysweep<ODR, FLUX, 8, MIX>(h, in, w, g); break;
-    }
-  } else {
-    launch_ysweep<ODR, FLUX, 8, MIX>(h, in, w, g);
-  }
+  const int ch = ychunk(h, g);
+  const dim3 gy((g.nx + 63) / 64, (g.ny - 5 + ch - 1) / ch);
+  if (split_march<MIX>(ch))
+    MLAU_LAUNCH(h, K_YSWEEP2D, (k_ysweep2d<ODR, FLUX, MIX, MIX != MLAU_FP64>), gy, dim3(64), in, w, g, ch);
+  else
+    MLAU_LAUNCH(h, K_YSWEEP2D, (k_ysweep2d<ODR, FLUX, MIX, false>), gy, dim3(64), in, w, g, ch);
   sd.leave();
   sd.join();
 }
@@ -212,17 +221,17 @@ static void stage2d(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const 
   MLAU_LAUNCH(h, K_BC2D, k_bc2d, dim3((unsigned)((nframe + 255) / 256), 8), b256, out, g, h->bc);
 }
 
-template <int ODR, int FLUX, int CH, int MIX>
-static void launch_ysweep_inl(Handle *h, const U2 &in, const W2 &w, const G2 &g)
+template <int ODR, int FLUX, int MIX, int CTW>
+static void launch_ysweep_inl(Handle *h, const U2 &in, const W2 &w, const G2 &g, dim3 gy, int ch)
 {
-  const dim3 gr((g.nx + 63) / 64, (g.ny - 5 + CH - 1) / CH);
-  if (h->s.ctw) MLAU_LAUNCH(h, K_YSW2D_INL, (k_ysweep2d_inl<ODR, FLUX, CH, MIX, 1>), gr, dim3(64), in, w, g);
-  else MLAU_LAUNCH(h, K_YSW2D_INL, (k_ysweep2d_inl<ODR, FLUX, CH, MIX, 0>), gr, dim3(64), in, w, g);
+  if (split_march<MIX>(ch))
+    MLAU_LAUNCH(h, K_YSW2D_INL, (k_ysweep2d_inl<ODR, FLUX, MIX, CTW, MIX != MLAU_FP64>), gy, dim3(64), in, w, g, ch);
+  else
+    MLAU_LAUNCH(h, K_YSW2D_INL, (k_ysweep2d_inl<ODR, FLUX, MIX, CTW, false>), gy, dim3(64), in, w, g, ch);
 }
 
 // Periodic grids (with room for the ghost images written by the update): the
-// stage without primitive arrays.  Tune bits 0-1 (ODR=4 with LHLLD only):
-// y-sweep chunk of 8 (default), 16 or 4 rows.
+// stage without primitive arrays.
 template <int ODR, int FLUX, int MIX>
 static void stage2d_inl(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const W2 &w, const G2 &g, double ra,
                         double rb)
@@ -232,15 +241,10 @@ static void stage2d_inl(Handle *h, const U2 &in, const U2 &ut, const U2 &out, co
   sd.fork(1);
   MLAU_LAUNCH(h, K_XSW2D_INL, (k_xsweep2d_inl<ODR, FLUX, MIX>), gx, dim3(256), in, w, g);
   sd.enter(0);
-  if constexpr (ODR == 4 && FLUX == FLUX_LHLLD) {  // the chunk variants for ODR=4 with LHLLD only
-    switch (h->tune & 3) {
-    case 1: launch_ysweep_inl<ODR, FLUX, 16, MIX>(h, in, w, g); break;
-    case 2: launch_ysweep_inl<ODR, FLUX, 4, MIX>(h, in, w, g); break;
-    default: launch_ysweep_inl<ODR, FLUX, 8, MIX>(h, in, w, g); break;
-    }
-  } else {
-    launch_ysweep_inl<ODR, FLUX, 8, MIX>(h, in, w, g);
-  }
+  const int ch = ychunk(h, g);
+  const dim3 gy((g.nx + 63) / 64, (g.ny - 5 + ch - 1) / ch);
+  if (h->s.ctw) launch_ysweep_inl<ODR, FLUX, MIX, 1>(h, in, w, g, gy, ch);
+  else launch_ysweep_inl<ODR, FLUX, MIX, 0>(h, in, w, g, gy, ch);
   sd.leave();
   sd.join();
   if (!h->s.ctw) {  // constant weight 1/2 (aux2d_body with CTW 0) over the corners the E-field reads

@@ -299,18 +299,22 @@ __device__ __forceinline__ void xsweep2d_body(U2 u, W2 w, G2 g, long wave, int l
 }
 
 // ----------------------------------------------------------------- ysweep2d
-// One lane per column i; each lane walks faces f0..f0+CH-1 (rows), carrying
+// One lane per column i; each lane walks faces f0..f0+ch-1 (rows), carrying
 // the left state of the face below from the previous iteration.
-// A 64-thread block (bx, by) holds columns 64*bx.. and faces 3+CH*by...
-template <int ODR, int FLUX, int CH, int MIX>
-__device__ __forceinline__ void ysweep2d_body(U2 u, W2 w, G2 g, unsigned bx, unsigned by, unsigned tid)
+// A 64-thread block (bx, by) holds columns 64*bx.. and faces 3+ch*by...
+// The cell below the first face is reconstructed ahead of the march (its left
+// state alone) or, with `mid`, as the march's first cell, by the code that the
+// later cells run (see march_mid).  SPLIT: whether `mid` may be set.
+template <int ODR, int FLUX, int MIX, bool SPLIT>
+__device__ __forceinline__ void ysweep2d_body(U2 u, W2 w, G2 g, int ch, bool mid, unsigned bx, unsigned by,
+                                              unsigned tid)
 {
   const int i = bx * 64 + tid;
   const int nx = g.nx, ny = g.ny;
   if (i >= nx) return;
-  const int f0 = 3 + CH * by;
+  const int f0 = 3 + ch * (int)by;
   if (f0 > ny - 3) return;
-  const int f1 = (f0 + CH - 1 < ny - 3) ? f0 + CH - 1 : ny - 3;
+  const int f1 = (f0 + ch - 1 < ny - 3) ? f0 + ch - 1 : ny - 3;
   // window rows r-2..r+2 of the rotated primitives (ro,vy,vz,vx,bz,cx,pr), m2
   double W[7][5], M[5];
   auto load = [&](int r, int m) {
@@ -343,11 +347,18 @@ __device__ __forceinline__ void ysweep2d_body(U2 u, W2 w, G2 g, unsigned bx, uns
     ql = a0 - u.f[6][q + nx] * a1;
     qr = b0 - u.f[6][q] * b1;
   };
-#pragma unroll
-  for (int m = 0; m < 5; m++) load(f0 - 3 + m, m);
   double vlp[7], vr[7], qlp, qr;
-  cell(f0 - 1, vlp, vr, qlp, qr);
-  for (int r = f0; r <= f1; r++) {
+  int r = f0;
+  if (SPLIT && mid) {
+    r = f0 - 1;
+#pragma unroll
+    for (int m = 1; m < 5; m++) load(f0 - 4 + m, m);
+  } else {
+#pragma unroll
+    for (int m = 0; m < 5; m++) load(f0 - 3 + m, m);
+    cell(f0 - 1, vlp, vr, qlp, qr);
+  }
+  for (; r <= f1; r++) {
 #pragma unroll
     for (int m = 0; m < 4; m++) {
 #pragma unroll
@@ -357,22 +368,24 @@ __device__ __forceinline__ void ysweep2d_body(U2 u, W2 w, G2 g, unsigned bx, uns
     load(r + 2, 4);
     double vl[7], ql;
     cell(r, vl, vr, ql, qr);
-    const long q = (long)r * nx + i;
-    const double byf = u.f[6][q];
-    const double bn = 0.5 * (byf + byf);
-    const double dv0 = w.vy[q] - w.vy[q - nx];
-    const double dv1 = dmin(w.dvx[q - nx], w.dvx[q]);
-    double f[7];
-    riemann_p<FLUX, MIX>(vlp, vr, bn, g.gamma, dv0, dv1, f);
-    const double fc = 0.5 * (qlp + qr);
-    w.fy[0][q] = f[0];
-    w.fy[1][q] = f[3];
-    w.fy[2][q] = f[1];
-    w.fy[3][q] = f[2];
-    w.fy[4][q] = f[5] - fc;
-    w.fy[5][q] = f[4];
-    w.fy[6][q] = f[6];
-    w.fcy[q] = fc;
+    if (!SPLIT || r >= f0) {
+      const long q = (long)r * nx + i;
+      const double byf = u.f[6][q];
+      const double bn = 0.5 * (byf + byf);
+      const double dv0 = w.vy[q] - w.vy[q - nx];
+      const double dv1 = dmin(w.dvx[q - nx], w.dvx[q]);
+      double f[7];
+      riemann_p<FLUX, MIX>(vlp, vr, bn, g.gamma, dv0, dv1, f);
+      const double fc = 0.5 * (qlp + qr);
+      w.fy[0][q] = f[0];
+      w.fy[1][q] = f[3];
+      w.fy[2][q] = f[1];
+      w.fy[3][q] = f[2];
+      w.fy[4][q] = f[5] - fc;
+      w.fy[5][q] = f[4];
+      w.fy[6][q] = f[6];
+      w.fcy[q] = fc;
+    }
 #pragma unroll
     for (int k = 0; k < 7; k++) vlp[k] = vl[k];
     qlp = ql;

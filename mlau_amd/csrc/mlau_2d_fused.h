@@ -95,17 +95,17 @@ __device__ __forceinline__ void xsweep2d_inl_body(const U2 &u, const W2 &w, cons
 // shuffles; the wavefront's two outermost lanes and ghost cells form it from
 // the state directly), and, with CTW, the CT weight of corner (i, f) (the
 // corners' rows are the faces').  Writes fy[0..6], fcy and ctx.  Periodic
-// grids.
-template <int ODR, int FLUX, int CH, int MIX, int CTW>
-__device__ __forceinline__ void ysweep2d_inl_body(const U2 &u, const W2 &w, const G2 &g, unsigned bx, unsigned by,
-                                                  unsigned lane)
+// grids.  `mid` and SPLIT as in ysweep2d_body.
+template <int ODR, int FLUX, int MIX, int CTW, bool SPLIT>
+__device__ __forceinline__ void ysweep2d_inl_body(const U2 &u, const W2 &w, const G2 &g, int ch, bool mid,
+                                                  unsigned bx, unsigned by, unsigned lane)
 {
   constexpr BcFlags bc{};  // periodic grids only: every boundary flag 0
   const int nx = g.nx, ny = g.ny;
   const long N = nx;
-  const int f0 = 3 + CH * by;
+  const int f0 = 3 + ch * (int)by;
   if (f0 > ny - 3) return;  // whole wavefront
-  const int f1 = (f0 + CH - 1 < ny - 3) ? f0 + CH - 1 : ny - 3;
+  const int f1 = (f0 + ch - 1 < ny - 3) ? f0 + ch - 1 : ny - 3;
   const int i = bx * 64 + lane;
   const bool live = i < nx;
   const int ic = live ? i : nx - 1;  // lanes past the grid take part in the shuffles only
@@ -157,12 +157,20 @@ __device__ __forceinline__ void ysweep2d_inl_body(const U2 &u, const W2 &w, cons
     ql = a0 - u.f[6][q + N] * a1;
     qr = b0 - u.f[6][q] * b1;
   };
-#pragma unroll
-  for (int m = 0; m < 5; m++) load(f0 - 3 + m, m);
   double vlp[7], vr[7], qlp, qr;
-  cell(f0 - 1, vlp, vr, qlp, qr);
-  double dvp = dvx(f0 - 1, 2);  // dvx of the row below the face (window row 1 after the shift)
-  for (int f = f0; f <= f1; f++) {
+  double dvp = 0.0;  // dvx of the row below the face (window row 1 after the shift)
+  int f = f0;
+  if (SPLIT && mid) {
+    f = f0 - 1;
+#pragma unroll
+    for (int m = 1; m < 5; m++) load(f0 - 4 + m, m);
+  } else {
+#pragma unroll
+    for (int m = 0; m < 5; m++) load(f0 - 3 + m, m);
+    cell(f0 - 1, vlp, vr, qlp, qr);
+    dvp = dvx(f0 - 1, 2);
+  }
+  for (; f <= f1; f++) {
 #pragma unroll
     for (int m = 0; m < 4; m++) {
 #pragma unroll
@@ -173,7 +181,7 @@ __device__ __forceinline__ void ysweep2d_inl_body(const U2 &u, const W2 &w, cons
     const double dvc = dvx(f, 2);
     const double dv1 = dmin(dvp, dvc);
     dvp = dvc;
-    if (CTW) {  // CT weight of corner (i, f) (aux2d_body), from rows f-1, f of columns i-1, i
+    if (CTW && (!SPLIT || f >= f0)) {  // CT weight of corner (i, f) (aux2d_body), from rows f-1, f of columns i-1, i
       double lvx1 = __shfl_up(W[3][1], 1, 64), lvy1 = __shfl_up(W[1][1], 1, 64), lro1 = __shfl_up(W[0][1], 1, 64);
       double lvx2 = __shfl_up(W[3][2], 1, 64), lvy2 = __shfl_up(W[1][2], 1, 64), lro2 = __shfl_up(W[0][2], 1, 64);
       const long q = (long)f * N + ic;
@@ -200,22 +208,24 @@ __device__ __forceinline__ void ysweep2d_inl_body(const U2 &u, const W2 &w, cons
     }
     double vl[7], ql;
     cell(f, vl, vr, ql, qr);
-    const long q = (long)f * N + ic;
-    const double byf = u.f[6][q];
-    const double bn = 0.5 * (byf + byf);
-    const double dv0 = W[1][2] - W[1][1];
-    double fl[7];
-    riemann_p<FLUX, MIX>(vlp, vr, bn, g.gamma, dv0, dv1, fl);
-    const double fc = 0.5 * (qlp + qr);
-    if (live) {
-      w.fy[0][q] = fl[0];
-      w.fy[1][q] = fl[3];
-      w.fy[2][q] = fl[1];
-      w.fy[3][q] = fl[2];
-      w.fy[4][q] = fl[5] - fc;
-      w.fy[5][q] = fl[4];
-      w.fy[6][q] = fl[6];
-      w.fcy[q] = fc;
+    if (!SPLIT || f >= f0) {
+      const long q = (long)f * N + ic;
+      const double byf = u.f[6][q];
+      const double bn = 0.5 * (byf + byf);
+      const double dv0 = W[1][2] - W[1][1];
+      double fl[7];
+      riemann_p<FLUX, MIX>(vlp, vr, bn, g.gamma, dv0, dv1, fl);
+      const double fc = 0.5 * (qlp + qr);
+      if (live) {
+        w.fy[0][q] = fl[0];
+        w.fy[1][q] = fl[3];
+        w.fy[2][q] = fl[1];
+        w.fy[3][q] = fl[2];
+        w.fy[4][q] = fl[5] - fc;
+        w.fy[5][q] = fl[4];
+        w.fy[6][q] = fl[6];
+        w.fcy[q] = fc;
+      }
     }
 #pragma unroll
     for (int k = 0; k < 7; k++) vlp[k] = vl[k];

@@ -17,6 +17,8 @@
 
 namespace mlau {
 
+constexpr int kMarch = 16;  // longest march of the y and z sweeps
+
 // Cell kernels: 1D grids of (plane pieces) x (planes or plane chunks), remapped
 // so that each XCD works on a contiguous band and neighbouring rows share its L2.
 struct Blk2 {
@@ -71,14 +73,15 @@ __global__ __launch_bounds__(256) void k_xsweep3d(Sw3 w, G3 g)
 
 // y/z sweeps: lanes over the flattened (i, third coordinate) columns; blocks
 // are (column piece, chunk along the sweep axis)
-template <int ODR, int FLUX, int CH, int AX, int MIX>
-__global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_msweep3d(Sw3 w, G3 g)
+template <int ODR, int FLUX, int AX, int MIX, bool SPLIT>
+__global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_msweep3d(Sw3 w, G3 g, int ch)
 {
   const long nc = (AX == 1) ? g.nz : g.ny;
   const unsigned pieces = (unsigned)((g.nx * nc + 63) / 64);
   const long p = (long)(blockIdx.x % pieces) * 64 + threadIdx.x;
   if (p >= g.nx * nc) return;
-  msweep3d_body<ODR, FLUX, CH, AX, MIX>(w, g, (int)(p % g.nx), blockIdx.x / pieces, (int)(p / g.nx));
+  const unsigned c = blockIdx.x / pieces;
+  msweep3d_body<ODR, FLUX, AX, MIX, SPLIT>(w, g, ch, march_mid(ch, c, kMarch), (int)(p % g.nx), c, (int)(p / g.nx));
 }
 
 template <int ODR>
@@ -134,7 +137,6 @@ __global__ __launch_bounds__(256) void k_cfl3d(U3 u, G3 g, StepInfo *info)
 }
 
 // ------------------------------------------------------------------- driver
-constexpr int kMChunk = 16;
 constexpr int kZChunk = 8;  // planes per thread of the z-marching edge/update kernels
 
 static G3 geom3(Handle *h)
@@ -169,6 +171,19 @@ static Sw3 sweep_view(Handle *h, const U3 &in, int ax)
   return w;
 }
 
+template <int ODR, int FLUX, int AX, int MIX>
+static void launch_march(Handle *h, int kid, const Sw3 &w, const G3 &g, long pieces, int faces, int ch)
+{
+  const dim3 gr((unsigned)(pieces * ((faces + ch - 1) / ch)));
+  if constexpr (MIX != MLAU_FP64) {
+    if (ch < kMarch) {
+      MLAU_LAUNCH(h, kid, (k_msweep3d<ODR, FLUX, AX, MIX, true>), gr, dim3(64), w, g, ch);
+      return;
+    }
+  }
+  MLAU_LAUNCH(h, kid, (k_msweep3d<ODR, FLUX, AX, MIX, false>), gr, dim3(64), w, g, ch);
+}
+
 template <int ODR, int FLUX, int MIX>
 static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double ra, double rb)
 {
@@ -194,18 +209,17 @@ static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double
   else
     MLAU_LAUNCH(h, K_AUX3D, (k_aux3d<0>), gflat, b256, in, (const double *)P[0], (const double *)P[1],
                 (const double *)P[2], h->aux[0], h->aux[1], h->aux[2], h->aux[3], h->aux[4], h->aux[5], g, h->bc);
+  const long xw = xsweep_waves((long)ny * nz, nx), yw = ((long)nx * nz + 63) / 64, zw = ((long)nx * ny + 63) / 64;
+  const int chy = march_chunk(yw, ny - 5, xw + zw * nz, 0.2, kMarch, MIX != MLAU_FP64);
+  const int chz = march_chunk(zw, nz - 5, xw + yw * ny, 0.2, kMarch, MIX != MLAU_FP64);
   Side sd(h);  // the y and z sweeps beside the x sweep
   sd.fork(2);
-  MLAU_LAUNCH(h, K_XSWEEP3D, (k_xsweep3d<ODR, FLUX, MIX>), dim3((unsigned)((xsweep_waves((long)ny * nz, nx) + 3) / 4)),
-              b256, sweep_view(h, in, 0), g);
+  MLAU_LAUNCH(h, K_XSWEEP3D, (k_xsweep3d<ODR, FLUX, MIX>), dim3((unsigned)((xw + 3) / 4)), b256,
+              sweep_view(h, in, 0), g);
   sd.enter(0);
-  MLAU_LAUNCH(h, K_YSWEEP3D, (k_msweep3d<ODR, FLUX, kMChunk, 1, MIX>),
-              dim3((unsigned)((((long)nx * nz + 63) / 64) * ((ny - 5 + kMChunk - 1) / kMChunk))), dim3(64),
-              sweep_view(h, in, 1), g);
+  launch_march<ODR, FLUX, 1, MIX>(h, K_YSWEEP3D, sweep_view(h, in, 1), g, yw, ny - 5, chy);
   sd.enter(1);
-  MLAU_LAUNCH(h, K_ZSWEEP3D, (k_msweep3d<ODR, FLUX, kMChunk, 2, MIX>),
-              dim3((unsigned)((((long)nx * ny + 63) / 64) * ((nz - 5 + kMChunk - 1) / kMChunk))), dim3(64),
-              sweep_view(h, in, 2), g);
+  launch_march<ODR, FLUX, 2, MIX>(h, K_ZSWEEP3D, sweep_view(h, in, 2), g, zw, nz - 5, chz);
   sd.leave();
   sd.join();
   Edge3 e;

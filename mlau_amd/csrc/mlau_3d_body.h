@@ -304,18 +304,18 @@ __device__ __forceinline__ void xsweep3d_body(const Sw3 &w, G3 g, long wave, int
 }
 
 // Y/Z sweep: one lane per column (i, bz) with bz the third coordinate (k for
-// Y, j for Z); the lane marches faces f0..f0+CH-1 (f0 = 3+CH*by) along the
-// sweep axis.
-template <int ODR, int FLUX, int CH, int AX, int MIX>
-__device__ __forceinline__ void msweep3d_body(const Sw3 &w, G3 g, int i, int by, int bz)
+// Y, j for Z); the lane marches faces f0..f0+ch-1 (f0 = 3+ch*by) along the
+// sweep axis; `mid` and SPLIT as in ysweep2d_body.
+template <int ODR, int FLUX, int AX, int MIX, bool SPLIT>
+__device__ __forceinline__ void msweep3d_body(const Sw3 &w, G3 g, int ch, bool mid, int i, int by, int bz)
 {
   const long nx = g.nx, nxy = (long)g.nx * g.ny;
   const int n = (AX == 1) ? g.ny : g.nz;
   const long st = (AX == 1) ? nx : nxy;
   const long base = (AX == 1) ? (long)bz * nxy + i : (long)bz * nx + i;
-  const int f0 = 3 + CH * by;
+  const int f0 = 3 + ch * by;
   if (f0 > n - 3) return;
-  const int f1 = (f0 + CH - 1 < n - 3) ? f0 + CH - 1 : n - 3;
+  const int f1 = (f0 + ch - 1 < n - 3) ? f0 + ch - 1 : n - 3;
   // window rows r-2..r+2 of cell r; bit m of supb: m2 >= 1 in window row m
   // (the reconstruction selector takes the maximum of rows r-1..r+1; for
   // finite values that is the same test)
@@ -344,11 +344,18 @@ __device__ __forceinline__ void msweep3d_body(const Sw3 &w, G3 g, int i, int by,
     central_lr<ODR>(W[4], W[1], W[2], w.bface[q + st], w.bface[q], qlt, qrt);
     central_lr<ODR>(W[5], W[1], W[3], w.bface[q + st], w.bface[q], qlu, qru);
   };
-#pragma unroll
-  for (int m = 0; m < 5; m++) load(f0 - 3 + m, m);
   double vlp[7], vr[7], qltp, qlup, qrt, qru;
-  cell(f0 - 1, vlp, vr, qltp, qrt, qlup, qru);
-  for (int r = f0; r <= f1; r++) {
+  int r = f0;
+  if (SPLIT && mid) {
+    r = f0 - 1;
+#pragma unroll
+    for (int m = 1; m < 5; m++) load(f0 - 4 + m, m);
+  } else {
+#pragma unroll
+    for (int m = 0; m < 5; m++) load(f0 - 3 + m, m);
+    cell(f0 - 1, vlp, vr, qltp, qrt, qlup, qru);
+  }
+  for (; r <= f1; r++) {
 #pragma unroll
     for (int m = 0; m < 4; m++) {
 #pragma unroll
@@ -358,7 +365,7 @@ __device__ __forceinline__ void msweep3d_body(const Sw3 &w, G3 g, int i, int by,
     load(r + 2, 4);
     double vl[7], qlt, qlu;
     cell(r, vl, vr, qlt, qrt, qlu, qru);
-    face_flux<FLUX, MIX>(w, base + r * st, st, vlp, vr, qltp, qlup, qrt, qru, g.gamma);
+    if (!SPLIT || r >= f0) face_flux<FLUX, MIX>(w, base + r * st, st, vlp, vr, qltp, qlup, qrt, qru, g.gamma);
 #pragma unroll
     for (int a = 0; a < 7; a++) vlp[a] = vl[a];
     qltp = qlt;

@@ -90,4 +90,47 @@ __device__ __forceinline__ void block_max_atomic(double v, unsigned long long *a
 // stride of 63 cells per 64-lane wavefront.
 __host__ __device__ __forceinline__ long xsweep_waves(long rows, int nx) { return (rows * (nx - 4) - 1 + 62) / 63; }
 
+// Faces per lane of a marching sweep (y in 2D, y and z in 3D).  A lane that
+// marches ch faces reconstructs ch+1 cells one after the other: a long march
+// wastes fewer reconstructions (1 in ch+1), a short one makes more wavefronts.
+// Times in units of one cell's issue time on a SIMD (6.1 us at WCNS4 + LHLLD):
+// the chip's 1024 SIMDs issue `pieces` columns of wavefronts marching the
+// faces plus the `others` wavefronts of the sweeps that run beside this one;
+// a wavefront with a SIMD to itself needs kLone of them per cell (7.5-9 us);
+// and at the end a SIMD idles for `tail` of a march on average, less in 3D where the two other
+// sweeps fill the gap.  Measured over 2D 64..2048 squared and 3D 24..128 cubed
+// (8 steps, us), fixed chunk 8 (2D) and 16 (3D) -> this choice:
+// 64^2 2268 -> 1045 (1 face), 256^2 2320 -> 1356 (1), 512^2 2774 -> 2497 (2), 768^2 4646 -> 4413 (4),
+// 2048^2 27159 (8), 32^3 6211 -> 3713 (1), 64^3 6905 -> 5729 (4), 128^3 29220 -> 29190 (8);
+// never more than 2 % above the best of 1, 2, 4, 8, 16.  `most` is 8 in 2D (16
+// gained nothing there at any size) and 16 in 3D.
+inline int march_chunk(long pieces, int faces, long others, double tail, int most, bool mixed)
+{
+  const double kSimds = 1024, kLone = 1.5;
+  int best = 1;
+  double least = 0.0;
+  for (int ch = 1; ch <= most; ch *= 2) {
+    const double cells = ch + (mixed && ch < most ? 1.6 : 1.0);  // a whole cell and a longer loop: march_mid
+    const double issue = ((double)(pieces * ((faces + ch - 1) / ch)) * cells + (double)others) / kSimds;
+    const double lone = kLone * (ch + 1);
+    const double t = issue + tail * lone > lone ? issue + tail * lone : lone;
+    if (ch == 1 || t < least) {
+      least = t;
+      best = ch;
+    }
+  }
+  return best;
+}
+
+// Whether a march that starts at face 3 + ch*c begins in the middle of a march
+// of `most` faces.  The left state of the cell below a march's first face
+// comes from a copy of the reconstruction that makes nothing else, in which the
+// compiler fuses other multiply-adds of the FP32 form than in the march's own
+// copy: the mixed forms therefore take that copy at the cells where the longest
+// march takes it and the march's own elsewhere, so that their results do not
+// depend on the march length.  FP64 fuses nothing and always takes the short
+// copy; so do longest marches, whose kernels are compiled without the choice
+// (with it the 128^3 mixed sweeps took 1 % longer).
+__device__ __forceinline__ bool march_mid(int ch, unsigned c, int most) { return (ch * c) % most != 0; }
+
 }  // namespace mlau

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_ens_ysweep2d(const EnsRec
   ENS_LOOP(T2_YSW)
     const U2 u = sin ? R.u1 : R.u0;
     const unsigned gyx = (R.g.nx + 63) / 64;
-    ysweep2d_body<ODR, FLUX, CH, MIX>(u, R.w, R.g, l_ % gyx, l_ / gyx, threadIdx.x);
+    ysweep2d_body<ODR, FLUX, MIX, false>(u, R.w, R.g, CH, false, l_ % gyx, l_ / gyx, threadIdx.x);
   }
 }
 

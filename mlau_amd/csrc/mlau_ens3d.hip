@@ -189,7 +189,7 @@ __global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_ens_msweep3d(const EnsRec
     const unsigned pieces = (unsigned)((R.g.nx * nc + 63) / 64);
     const long p = (long)(l_ % pieces) * 64 + threadIdx.x;
     if (p >= R.g.nx * nc) continue;
-    msweep3d_body<ODR, FLUX, kEnsMChunk, AX, MIX>(w, R.g, (int)(p % R.g.nx), l_ / pieces, (int)(p / R.g.nx));
+    msweep3d_body<ODR, FLUX, AX, MIX, false>(w, R.g, kEnsMChunk, false, (int)(p % R.g.nx), l_ / pieces, (int)(p / R.g.nx));
   }
 }
 
