@@ -65,7 +65,8 @@ __global__ __launch_bounds__(256) void k_stage1d(U1d in, U1d ut, U1d out, G1d g,
   }
 }
 
-__global__ __launch_bounds__(256) void k_cfl1d(U1d u, G1d g, StepInfo *info)
+__global__ __launch_bounds__(256) void k_cfl1d(U1d u, G1d g, StepInfo *info, double cfl, double vfloor,
+                                               double dx, double dy, double dz)
 {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   double v = 0.0;
@@ -73,7 +74,8 @@ __global__ __launch_bounds__(256) void k_cfl1d(U1d u, G1d g, StepInfo *info)
     const double vt = cfl1d_cell(u, g, i);
     if (vt > v) v = vt;
   }
-  block_max_atomic<256>(v, &info->vmax_bits);
+  v = block_max<256>(v);
+  if (threadIdx.x == 0) cfl_finish(info, v, cfl, vfloor, dx, dx, dy, dz);
 }
 
 static void views1d(Handle *h, U1d &u0, U1d &u1, W1d &w, G1d &g)
@@ -169,10 +171,8 @@ int run_cfl_1d(Handle *h, double cfl, double vfloor)
   W1d w;
   G1d g;
   views1d(h, u0, u1, w, g);
-  hipLaunchKernelGGL(k_cfl_reset, dim3(1), dim3(1), 0, h->stream, h->info, vfloor);
-  MLAU_LAUNCH(h, K_CFL1D, k_cfl1d, dim3((g.nx + 255) / 256), dim3(256), u0, g, h->info);
-  hipLaunchKernelGGL(k_finalize_dt, dim3(1), dim3(1), 0, h->stream, h->info, cfl, h->g.dx, h->g.dx, h->g.dy,
-                     h->g.dz);
+  MLAU_LAUNCH(h, K_CFL1D, k_cfl1d, dim3((g.nx + 255) / 256), dim3(256), u0, g, h->info, cfl, vfloor, h->g.dx, h->g.dy,
+              h->g.dz);
   return (int)hipGetLastError();
 }
 

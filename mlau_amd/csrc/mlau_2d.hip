@@ -74,18 +74,20 @@ __global__ __launch_bounds__(256) void k_ez2d(W2 w, G2 g)
 }
 
 template <int ODR, bool FIRST>
-__global__ __launch_bounds__(256) void k_update2d(U2 in, U2 ut, U2 out, W2 w, G2 g, const StepInfo *info,
-                                                  double ra, double rb)
+__global__ __launch_bounds__(256) void k_update2d(U2 in, U2 ut, U2 out, W2 w, G2 g, StepInfo *info, double ra,
+                                                  double rb, int adv)
 {
+  if (adv) advance_time(info);
   REGION_CELL(g.nx - 2 * g.xoff + 1, g.ny - 2 * g.yoff + 1, g.xoff, g.yoff)
   update2d_body<ODR, FIRST>(in, ut, out, w, g, info->dtdx, info->dtdy, ra, rb, i, j);
 }
 
 // periodic grids: interior cells, ghost images written with them (no k_bc2d)
 template <int ODR, bool FIRST>
-__global__ __launch_bounds__(256) void k_update2d_per(U2 in, U2 ut, U2 out, W2 w, G2 g, const StepInfo *info,
-                                                      double ra, double rb)
+__global__ __launch_bounds__(256) void k_update2d_per(U2 in, U2 ut, U2 out, W2 w, G2 g, StepInfo *info, double ra,
+                                                      double rb, int adv)
 {
+  if (adv) advance_time(info);
   REGION_CELL(g.nx - 2 * g.xoff, g.ny - 2 * g.yoff, g.xoff, g.yoff)
   update2d_body<ODR, FIRST, true>(in, ut, out, w, g, info->dtdx, info->dtdy, ra, rb, i, j);
 }
@@ -115,13 +117,15 @@ __global__ __launch_bounds__(256) void k_ctx_half2d(W2 w, G2 g)
 }
 
 // blockIdx.y = field
-__global__ __launch_bounds__(256) void k_bc2d(U2 u, G2 g, BcFlags bc)
+__global__ __launch_bounds__(256) void k_bc2d(U2 u, G2 g, BcPack bc)
 {
-  bc2d_body(u, g, bc, blockIdx.y, (long)blockIdx.x * blockDim.x + threadIdx.x);
+  const BcField b = bc_field(u.f, bc, blockIdx.y);
+  bc2d_body(b, g, (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // vmax over the interior, grid-stride with one atomic per block.
-__global__ __launch_bounds__(256) void k_cfl2d(U2 u, G2 g, StepInfo *info)
+__global__ __launch_bounds__(256) void k_cfl2d(U2 u, G2 g, StepInfo *info, double cfl, double vfloor,
+                                               double dr, double dx, double dy, double dz)
 {
   const long total = (long)(g.nx - 2 * g.xoff) * (g.ny - 2 * g.yoff);
   double v = 0.0;
@@ -129,7 +133,8 @@ __global__ __launch_bounds__(256) void k_cfl2d(U2 u, G2 g, StepInfo *info)
     const double vt = cfl2d_cell(u, g, t);
     if (vt > v) v = vt;
   }
-  block_max_atomic<256>(v, &info->vmax_bits);
+  v = block_max<256>(v);
+  if (threadIdx.x == 0) cfl_finish(info, v, cfl, vfloor, dr, dx, dy, dz);
 }
 
 // ------------------------------------------------------------------ driver
@@ -189,7 +194,7 @@ static void sweeps2d(Handle *h, const U2 &in, const W2 &w, const G2 &g)
 
 template <int ODR, int FLUX, int MIX>
 static void stage2d(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const W2 &w, const G2 &g, double ra,
-                    double rb)
+                    double rb, int adv)
 {
   const int nx = g.nx, ny = g.ny;
   dim3 b256(256);
@@ -207,18 +212,17 @@ static void stage2d(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const 
   MLAU_LAUNCH(h, K_EZ2D, (k_ez2d<ODR>), dim3(region_pieces(nx - 5, ny - 5)), b256, w, g);
   if (h->periodic_images && !(h->tune & 16)) {  // tune bit 4: separate boundary pass
     const dim3 gp(region_pieces(nx - 2 * g.xoff, ny - 2 * g.yoff));
-    const StepInfo *info = h->info;
-    if (ra == 0.0) MLAU_LAUNCH(h, K_UPD2D, (k_update2d_per<ODR, true>), gp, b256, in, ut, out, w, g, info, ra, rb);
-    else MLAU_LAUNCH(h, K_UPD2D, (k_update2d_per<ODR, false>), gp, b256, in, ut, out, w, g, info, ra, rb);
+    if (ra == 0.0) MLAU_LAUNCH(h, K_UPD2D, (k_update2d_per<ODR, true>), gp, b256, in, ut, out, w, g, h->info, ra, rb, adv);
+    else MLAU_LAUNCH(h, K_UPD2D, (k_update2d_per<ODR, false>), gp, b256, in, ut, out, w, g, h->info, ra, rb, adv);
     return;
   }
   const dim3 gu(region_pieces(nx - 2 * g.xoff + 1, ny - 2 * g.yoff + 1));
   if (ra == 0.0)
-    MLAU_LAUNCH(h, K_UPD2D, (k_update2d<ODR, true>), gu, b256, in, ut, out, w, g, (const StepInfo *)h->info, ra, rb);
+    MLAU_LAUNCH(h, K_UPD2D, (k_update2d<ODR, true>), gu, b256, in, ut, out, w, g, h->info, ra, rb, adv);
   else
-    MLAU_LAUNCH(h, K_UPD2D, (k_update2d<ODR, false>), gu, b256, in, ut, out, w, g, (const StepInfo *)h->info, ra, rb);
+    MLAU_LAUNCH(h, K_UPD2D, (k_update2d<ODR, false>), gu, b256, in, ut, out, w, g, h->info, ra, rb, adv);
   const long nframe = (long)ny * 2 * g.xoff + (long)2 * g.yoff * nx;
-  MLAU_LAUNCH(h, K_BC2D, k_bc2d, dim3((unsigned)((nframe + 255) / 256), 8), b256, out, g, h->bc);
+  MLAU_LAUNCH(h, K_BC2D, k_bc2d, dim3((unsigned)((nframe + 255) / 256), 8), b256, out, g, bc_pack(h->bc));
 }
 
 template <int ODR, int FLUX, int MIX, int CTW>
@@ -234,7 +238,7 @@ static void launch_ysweep_inl(Handle *h, const U2 &in, const W2 &w, const G2 &g,
 // stage without primitive arrays.
 template <int ODR, int FLUX, int MIX>
 static void stage2d_inl(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const W2 &w, const G2 &g, double ra,
-                        double rb)
+                        double rb, int adv)
 {
   const dim3 gx((unsigned)((xsweep_waves(g.ny, g.nx) + 3) / 4));
   Side sd(h);  // the y sweep beside the x sweep
@@ -253,9 +257,8 @@ static void stage2d_inl(Handle *h, const U2 &in, const U2 &ut, const U2 &out, co
   }
   MLAU_LAUNCH(h, K_EZ2D, (k_ez2d<ODR>), dim3(region_pieces(g.nx - 5, g.ny - 5)), dim3(256), w, g);
   const dim3 gp(region_pieces(g.nx - 2 * g.xoff, g.ny - 2 * g.yoff));
-  const StepInfo *info = h->info;
-  if (ra == 0.0) MLAU_LAUNCH(h, K_UPD2D, (k_update2d_per<ODR, true>), gp, dim3(256), in, ut, out, w, g, info, ra, rb);
-  else MLAU_LAUNCH(h, K_UPD2D, (k_update2d_per<ODR, false>), gp, dim3(256), in, ut, out, w, g, info, ra, rb);
+  if (ra == 0.0) MLAU_LAUNCH(h, K_UPD2D, (k_update2d_per<ODR, true>), gp, dim3(256), in, ut, out, w, g, h->info, ra, rb, adv);
+  else MLAU_LAUNCH(h, K_UPD2D, (k_update2d_per<ODR, false>), gp, dim3(256), in, ut, out, w, g, h->info, ra, rb, adv);
 }
 
 // The stage without primitive arrays applies to periodic grids whose interior
@@ -276,8 +279,9 @@ static void step2d(Handle *h)
   for (int rk = 0; rk < R_K; rk++) {
     const U2 &in = (rk == 0) ? u0 : u1;
     const U2 &out = (rk == R_K - 1) ? u0 : u1;
-    if (inl) stage2d_inl<ODR, FLUX, MIX>(h, in, u0, out, w, g, rkf[rk][0], rkf[rk][1]);
-    else stage2d<ODR, FLUX, MIX>(h, in, u0, out, w, g, rkf[rk][0], rkf[rk][1]);
+    const int adv = rk == R_K - 1;
+    if (inl) stage2d_inl<ODR, FLUX, MIX>(h, in, u0, out, w, g, rkf[rk][0], rkf[rk][1], adv);
+    else stage2d<ODR, FLUX, MIX>(h, in, u0, out, w, g, rkf[rk][0], rkf[rk][1], adv);
   }
 }
 
@@ -308,12 +312,10 @@ int run_cfl_2d(Handle *h, double cfl, double vfloor)
   W2 w;
   G2 g;
   make_views(h, u0, u1, w, g);
-  hipLaunchKernelGGL(k_cfl_reset, dim3(1), dim3(1), 0, h->stream, h->info, vfloor);
   const long cells = (long)(g.nx - 2 * g.xoff) * (g.ny - 2 * g.yoff);
-  const unsigned nb = (unsigned)((cells + 255) / 256 < 2048 ? (cells + 255) / 256 : 2048);
-  MLAU_LAUNCH(h, K_CFL2D, k_cfl2d, dim3(nb), dim3(256), u0, g, h->info);
+  const unsigned nb = cfl_blocks(cells);
   const double dr = (h->g.dx < h->g.dy) ? h->g.dx : h->g.dy;
-  hipLaunchKernelGGL(k_finalize_dt, dim3(1), dim3(1), 0, h->stream, h->info, cfl, dr, h->g.dx, h->g.dy, h->g.dz);
+  MLAU_LAUNCH(h, K_CFL2D, k_cfl2d, dim3(nb), dim3(256), u0, g, h->info, cfl, vfloor, dr, h->g.dx, h->g.dy, h->g.dz);
   return (int)hipGetLastError();
 }
 
@@ -327,8 +329,7 @@ int run_steps_2d(Handle *h, int nsteps, bool cfl_mode, double cfl, double vfloor
   default: fn = pick2<4>(h->s.flux, h->s.precision); break;
   }
   for (int n = 0; n < nsteps; n++) {
-    fn(h);
-    hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(1), 0, h->stream, h->info);
+    fn(h);  // its last update advances the time
     if (cfl_mode) run_cfl_2d(h, cfl, vfloor);
   }
   return (int)hipGetLastError();

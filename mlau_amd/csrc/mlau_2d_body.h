@@ -490,10 +490,10 @@ __device__ __forceinline__ void update2d_body(U2 in, U2 ut, U2 out, W2 w, G2 g,
 }
 
 // --------------------------------------------------------------------- bc2d
-// Ghost frame of field fld, frame point t: first the 2*xoff ghost columns of
+// Ghost frame of a field, frame point t: first the 2*xoff ghost columns of
 // every row, then the 2*yoff ghost rows.
 __device__ __forceinline__ long bc2d_points(G2 g) { return (long)g.ny * 2 * g.xoff + (long)2 * g.yoff * g.nx; }
-__device__ __forceinline__ void bc2d_body(U2 u, G2 g, const BcFlags &bc, int fld, long t)
+__device__ __forceinline__ void bc2d_body(const BcField &b, G2 g, long t)
 {
   const int nx = g.nx, ny = g.ny, xo = g.xoff, yo = g.yoff;
   const long nxs = (long)ny * 2 * xo;
@@ -510,10 +510,10 @@ __device__ __forceinline__ void bc2d_body(U2 u, G2 g, const BcFlags &bc, int fld
     j = (k < yo) ? k : ny - 2 * yo + k;
   }
   double sg = 1.0;
-  const int si = bc_src(i, nx, xo, bc.stx[fld], bc.dnx[fld], &sg);
-  const int sj = bc_src(j, ny, yo, bc.sty[fld], bc.dny[fld], &sg);
+  const int si = bc_src(i, nx, xo, b.stx, b.dnx, &sg);
+  const int sj = bc_src(j, ny, yo, b.sty, b.dny, &sg);
   if (si == i && sj == j) return;  // a face the solver itself updated
-  double *f = u.f[fld];
+  double *f = b.f;
   f[(long)j * nx + i] = sg * f[(long)sj * nx + si];
 }
 

@@ -101,9 +101,10 @@ __global__ __launch_bounds__(256) void k_edge3d_zm(Edge3 e, G3 g)
 
 template <int ODR, int CZ>
 __global__ __launch_bounds__(256) void k_update3d_zm(U3 in, U3 ut, U3 out, Fl3 fl, const double *ex,
-                                                     const double *ey, const double *ez, G3 g, const StepInfo *info,
-                                                     double ra, double rb)
+                                                     const double *ey, const double *ez, G3 g, StepInfo *info, double ra,
+                                                     double rb, int adv)
 {
+  if (adv) advance_time(info);
   const Blk2 b = banded2(plane_pieces(g.nx - 2 * g.xoff + 1, g.ny - 2 * g.yoff + 1));
   int i, j;
   if (!plane_face_cell(g, b.piece, threadIdx.x, i, j)) return;
@@ -113,19 +114,22 @@ __global__ __launch_bounds__(256) void k_update3d_zm(U3 in, U3 ut, U3 out, Fl3 f
 
 template <int ODR>
 __global__ __launch_bounds__(256) void k_update3d(U3 in, U3 ut, U3 out, Fl3 fl, const double *ex, const double *ey,
-                                                  const double *ez, G3 g, const StepInfo *info, double ra, double rb)
+                                                  const double *ez, G3 g, StepInfo *info, double ra, double rb, int adv)
 {
+  if (adv && blockIdx.y == 0 && blockIdx.z == 0) advance_time(info);
   update3d_body<ODR>(in, ut, out, fl, ex, ey, ez, g, info->dtdx, info->dtdy, info->dtdz, ra, rb, blockIdx.x,
                      blockIdx.y, blockIdx.z, threadIdx.x);
 }
 
 // blockIdx.y = field
-__global__ __launch_bounds__(256) void k_bc3d(U3 u, G3 g, BcFlags bc)
+__global__ __launch_bounds__(256) void k_bc3d(U3 u, G3 g, BcPack bc)
 {
-  bc3d_body(u, g, bc, blockIdx.y, (long)blockIdx.x * blockDim.x + threadIdx.x);
+  const BcField b = bc_field(u.f, bc, blockIdx.y);
+  bc3d_body(b, g, (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-__global__ __launch_bounds__(256) void k_cfl3d(U3 u, G3 g, StepInfo *info)
+__global__ __launch_bounds__(256) void k_cfl3d(U3 u, G3 g, StepInfo *info, double cfl, double vfloor,
+                                               double dr, double dx, double dy, double dz)
 {
   const long total = (long)(g.nx - 2 * g.xoff) * (g.ny - 2 * g.yoff) * (g.nz - 2 * g.zoff);
   double v = 0.0;
@@ -133,7 +137,8 @@ __global__ __launch_bounds__(256) void k_cfl3d(U3 u, G3 g, StepInfo *info)
     const double vt = cfl3d_cell(u, g, t);
     if (vt > v) v = vt;
   }
-  block_max_atomic<256>(v, &info->vmax_bits);
+  v = block_max<256>(v);
+  if (threadIdx.x == 0) cfl_finish(info, v, cfl, vfloor, dr, dx, dy, dz);
 }
 
 // ------------------------------------------------------------------- driver
@@ -185,7 +190,7 @@ static void launch_march(Handle *h, int kid, const Sw3 &w, const G3 &g, long pie
 }
 
 template <int ODR, int FLUX, int MIX>
-static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double ra, double rb)
+static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double ra, double rb, int adv)
 {
   const G3 g = geom3(h);
   const int nx = g.nx, ny = g.ny, nz = g.nz;
@@ -244,14 +249,14 @@ static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double
                 dim3(plane_pieces(nx - 2 * g.xoff + 1, ny - 2 * g.yoff + 1) *
                      ((nz - 2 * g.zoff + 1 + kZChunk - 1) / kZChunk)),
                 b256, in, ut, out, fl, (const double *)h->e[0], (const double *)h->e[1], (const double *)h->e[2], g,
-                (const StepInfo *)h->info, ra, rb);
+                h->info, ra, rb, adv);
   else
     MLAU_LAUNCH(h, K_UPD3D, (k_update3d<ODR>),
                 dim3((nx - 2 * g.xoff + 1 + 255) / 256, ny - 2 * g.yoff + 1, nz - 2 * g.zoff + 1), b256, in, ut, out,
                 fl, (const double *)h->e[0], (const double *)h->e[1], (const double *)h->e[2], g,
-                (const StepInfo *)h->info, ra, rb);
+                h->info, ra, rb, adv);
   const long nslab = (long)2 * g.xoff * ny * nz + (long)nx * 2 * g.yoff * nz + (long)nx * ny * 2 * g.zoff;
-  MLAU_LAUNCH(h, K_BC3D, k_bc3d, dim3((unsigned)((nslab + 255) / 256), 8), b256, out, g, h->bc);
+  MLAU_LAUNCH(h, K_BC3D, k_bc3d, dim3((unsigned)((nslab + 255) / 256), 8), b256, out, g, bc_pack(h->bc));
 }
 
 template <int ODR, int FLUX, int MIX>
@@ -267,7 +272,7 @@ static void step3d(Handle *h)
   for (int rk = 0; rk < R_K; rk++) {
     const U3 &in = (rk == 0) ? u0 : u1;
     const U3 &out = (rk == R_K - 1) ? u0 : u1;
-    stage3d<ODR, FLUX, MIX>(h, in, u0, out, rkf[rk][0], rkf[rk][1]);
+    stage3d<ODR, FLUX, MIX>(h, in, u0, out, rkf[rk][0], rkf[rk][1], rk == R_K - 1);
   }
 }
 
@@ -297,14 +302,12 @@ int run_cfl_3d(Handle *h, double cfl, double vfloor)
   const G3 g = geom3(h);
   U3 u0;
   for (int n = 0; n < 8; n++) u0.f[n] = h->U0[n];
-  hipLaunchKernelGGL(k_cfl_reset, dim3(1), dim3(1), 0, h->stream, h->info, vfloor);
   const long cells = (long)(g.nx - 2 * g.xoff) * (g.ny - 2 * g.yoff) * (g.nz - 2 * g.zoff);
-  const unsigned nb = (unsigned)((cells + 255) / 256 < 2048 ? (cells + 255) / 256 : 2048);
-  MLAU_LAUNCH(h, K_CFL3D, k_cfl3d, dim3(nb), dim3(256), u0, g, h->info);
+  const unsigned nb = cfl_blocks(cells);
   double dr = h->g.dx;
   if (h->g.dy < dr) dr = h->g.dy;
   if (h->g.dz < dr) dr = h->g.dz;
-  hipLaunchKernelGGL(k_finalize_dt, dim3(1), dim3(1), 0, h->stream, h->info, cfl, dr, h->g.dx, h->g.dy, h->g.dz);
+  MLAU_LAUNCH(h, K_CFL3D, k_cfl3d, dim3(nb), dim3(256), u0, g, h->info, cfl, vfloor, dr, h->g.dx, h->g.dy, h->g.dz);
   return (int)hipGetLastError();
 }
 
@@ -318,8 +321,7 @@ int run_steps_3d(Handle *h, int nsteps, bool cfl_mode, double cfl, double vfloor
   default: fn = pick3<4>(h->s.flux, h->s.precision); break;
   }
   for (int n = 0; n < nsteps; n++) {
-    fn(h);
-    hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(1), 0, h->stream, h->info);
+    fn(h);  // its last update advances the time
     if (cfl_mode) run_cfl_3d(h, cfl, vfloor);
   }
   return (int)hipGetLastError();

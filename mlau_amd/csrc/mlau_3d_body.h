@@ -655,7 +655,7 @@ __device__ __forceinline__ long bc3d_points(G3 g)
 {
   return (long)2 * g.xoff * g.ny * g.nz + (long)g.nx * 2 * g.yoff * g.nz + (long)g.nx * g.ny * 2 * g.zoff;
 }
-__device__ __forceinline__ void bc3d_body(U3 u, G3 g, const BcFlags &bc, int fld, long t)
+__device__ __forceinline__ void bc3d_body(const BcField &b, G3 g, long t)
 {
   const int nx = g.nx, ny = g.ny, nz = g.nz, xo = g.xoff, yo = g.yoff, zo = g.zoff;
   const long sx = (long)2 * xo * ny * nz, sy = (long)nx * 2 * yo * nz, sz = (long)nx * ny * 2 * zo;
@@ -682,11 +682,11 @@ __device__ __forceinline__ void bc3d_body(U3 u, G3 g, const BcFlags &bc, int fld
     return;
   }
   double sg = 1.0;
-  const int si = bc_src(i, nx, xo, bc.stx[fld], bc.dnx[fld], &sg);
-  const int sj = bc_src(j, ny, yo, bc.sty[fld], bc.dny[fld], &sg);
-  const int sk = bc_src(k, nz, zo, bc.stz[fld], bc.dnz[fld], &sg);
+  const int si = bc_src(i, nx, xo, b.stx, b.dnx, &sg);
+  const int sj = bc_src(j, ny, yo, b.sty, b.dny, &sg);
+  const int sk = bc_src(k, nz, zo, b.stz, b.dnz, &sg);
   if (si == i && sj == j && sk == k) return;
-  double *f = u.f[fld];
+  double *f = b.f;
   const long NX = nx, NXY = (long)nx * ny;
   f[k * NXY + j * NX + i] = sg * f[sk * NXY + sj * NX + si];
 }

@@ -36,27 +36,6 @@ int hip_fail(hipError_t e, const char *where)
     if (_e != hipSuccess) return hip_fail(_e, #call); \
   } while (0)
 
-__global__ void k_finalize_dt(StepInfo *info, double cfl, double dr, double dx, double dy, double dz)
-{
-  const double vmax = __longlong_as_double((long long)info->vmax_bits);
-  info->vmax = vmax;
-  if (isfinite(vmax)) {
-    const double dt = cfl * dr / vmax;
-    info->dt = dt;
-    info->dtdx = dt / dx;
-    info->dtdy = dt / dy;
-    info->dtdz = dt / dz;
-  }
-}
-__global__ void k_cfl_reset(StepInfo *info, double vfloor)
-{
-  info->vmax_bits = (unsigned long long)__double_as_longlong(vfloor);
-}
-__global__ void k_advance_time(StepInfo *info)
-{
-  info->tim += info->dt;
-  info->nstep += 1;
-}
 __global__ void k_set_time(StepInfo *info, double tim, long long nstep)
 {
   info->tim = tim;

@@ -219,7 +219,9 @@ __global__ __launch_bounds__(256) void k_ens_bc2d(const EnsRec2D *__restrict__ r
   ENS_LOOP(T2_BC)
     const unsigned nbf = (unsigned)((bc2d_points(R.g) + 255) / 256);
     const int fld = l_ / nbf;
-    bc2d_body(ubuf2(R, sout), R.g, R.bc, fld, (long)(l_ % nbf) * 256 + threadIdx.x);
+    const U2 &U = sout == 0 ? R.u0 : sout == 1 ? R.u1 : R.u2;
+    const BcField b{U.f[fld], R.bc.dnx[fld], R.bc.dny[fld], 0, R.bc.stx[fld], R.bc.sty[fld], 0};
+    bc2d_body(b, R.g, (long)(l_ % nbf) * 256 + threadIdx.x);
   }
 }
 

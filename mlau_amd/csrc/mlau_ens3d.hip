@@ -241,7 +241,9 @@ __global__ __launch_bounds__(256) void k_ens_bc3d(const EnsRec3D *__restrict__ r
   ENS_LOOP(T3_BC)
     const unsigned nbf = (unsigned)((bc3d_points(R.g) + 255) / 256);
     const int fld = l_ / nbf;
-    bc3d_body(sout ? R.u1 : R.u0, R.g, R.bc, fld, (long)(l_ % nbf) * 256 + threadIdx.x);
+    const U3 &U = sout ? R.u1 : R.u0;
+    const BcField b{U.f[fld], R.bc.dnx[fld], R.bc.dny[fld], R.bc.dnz[fld], R.bc.stx[fld], R.bc.sty[fld], R.bc.stz[fld]};
+    bc3d_body(b, R.g, (long)(l_ % nbf) * 256 + threadIdx.x);
   }
 }
 #undef CELL_COORDS

@@ -34,6 +34,42 @@ struct BcFlags {
   int stx[8], sty[8], stz[8];
 };
 
+// Array and flags of one field.
+struct BcField {
+  double *f;
+  int dnx, dny, dnz, stx, sty, stz;
+};
+// The flags of all fields as kernel arguments: two bits per field (dn + 1).
+struct BcPack {
+  unsigned x, y, z;
+};
+inline BcPack bc_pack(const BcFlags &bc)
+{
+  BcPack p{0, 0, 0};
+  for (int n = 0; n < 8; n++) {
+    p.x |= (unsigned)(bc.dnx[n] + 1) << (2 * n);
+    p.y |= (unsigned)(bc.dny[n] + 1) << (2 * n);
+    p.z |= (unsigned)(bc.dnz[n] + 1) << (2 * n);
+  }
+  return p;
+}
+// Field fld (the same in all threads of a block) out of kernel arguments.  A
+// run-time index into arrays of arguments makes every thread copy them to LDS or
+// scratch first (the 515x391 frame took 17 us instead of 6); the pointers pass
+// through an empty asm so that their selects stay selects of scalar registers.
+__device__ __forceinline__ BcField bc_field(double *const (&f)[8], BcPack p, int fld)
+{
+  double *at = nullptr;
+#pragma unroll
+  for (int n = 0; n < 8; n++) {
+    double *a = f[n];
+    asm("" : "+s"(a));
+    at = fld == n ? a : at;
+  }
+  return BcField{at, (int)(p.x >> (2 * fld) & 3u) - 1, (int)(p.y >> (2 * fld) & 3u) - 1,
+                 (int)(p.z >> (2 * fld) & 3u) - 1, fld == 5, fld == 6, fld == 7};
+}
+
 struct Handle {
   mlau_grid g;
   mlau_scheme s;
@@ -123,10 +159,6 @@ int run_cfl_1d(Handle *h, double cfl, double vfloor);
 int run_cfl_2d(Handle *h, double cfl, double vfloor);
 int run_cfl_3d(Handle *h, double cfl, double vfloor);
 
-// Device-side dt update from the reduced vmax: dt = cfl*dr/vmax when finite.
-__global__ void k_finalize_dt(StepInfo *info, double cfl, double dr, double dx, double dy, double dz);
-__global__ void k_cfl_reset(StepInfo *info, double vfloor);
-__global__ void k_advance_time(StepInfo *info);
 __global__ void k_set_dt(StepInfo *info, double dt, double dx, double dy, double dz);
 
 // Argument checks of mlau_create (grid and scheme).
