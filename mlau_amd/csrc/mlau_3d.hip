@@ -51,15 +51,15 @@ __global__ __launch_bounds__(256) void k_aux3d(U3 u, const double *vx, const dou
   aux3d_body<CTW>(u, vx, vy, vz, ct0, ct1, ct2, dvx, dvy, dvz, g, bc, i, j, b.plane);
 }
 
-template <int CTW, int CZ>
-__global__ __launch_bounds__(256) void k_aux3d_zm(U3 u, const double *vx, const double *vy, const double *vz,
+template <int CTW>
+__global__ __launch_bounds__(256) void k_aux3d_zm(int cz, U3 u, const double *vx, const double *vy, const double *vz,
                                                   double *ct0, double *ct1, double *ct2, double *dvx, double *dvy,
                                                   double *dvz, G3 g, BcFlags bc)
 {
   const Blk2 b = banded2(plane_pieces(g.nx, g.ny));
   int i, j;
   if (!plane_cell(g, b.piece, threadIdx.x, i, j)) return;
-  aux3d_zm_body<CTW, CZ>(u, vx, vy, vz, ct0, ct1, ct2, dvx, dvy, dvz, g, bc, i, j, b.plane);
+  aux3d_zm_body<CTW>(cz, u, vx, vy, vz, ct0, ct1, ct2, dvx, dvy, dvz, g, bc, i, j, b.plane);
 }
 
 // x sweep: row-flattened wavefronts, 4 per block
@@ -90,17 +90,18 @@ __global__ __launch_bounds__(256) void k_edge3d(Edge3 e, G3 g)
   edge3d_body<ODR>(e, g, blockIdx.x, blockIdx.y, blockIdx.z, threadIdx.x);
 }
 
+// CZ: planes per thread, 0 for `cz` of them
 template <int ODR, int CZ>
-__global__ __launch_bounds__(256) void k_edge3d_zm(Edge3 e, G3 g)
+__global__ __launch_bounds__(256) void k_edge3d_zm(int cz, Edge3 e, G3 g)
 {
   const Blk2 b = banded2(plane_pieces(g.nx, g.ny));
   int i, j;
   if (!plane_cell(g, b.piece, threadIdx.x, i, j)) return;
-  edge3d_zm_body<ODR, CZ>(e, g, i, j, b.plane);
+  edge3d_zm_body<ODR>(CZ ? CZ : cz, e, g, i, j, b.plane);
 }
 
 template <int ODR, int CZ>
-__global__ __launch_bounds__(256) void k_update3d_zm(U3 in, U3 ut, U3 out, Fl3 fl, const double *ex,
+__global__ __launch_bounds__(256) void k_update3d_zm(int cz, U3 in, U3 ut, U3 out, Fl3 fl, const double *ex,
                                                      const double *ey, const double *ez, G3 g, StepInfo *info, double ra,
                                                      double rb, int adv)
 {
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(256) void k_update3d_zm(U3 in, U3 ut, U3 out, Fl3 f
   const Blk2 b = banded2(plane_pieces(g.nx - 2 * g.xoff + 1, g.ny - 2 * g.yoff + 1));
   int i, j;
   if (!plane_face_cell(g, b.piece, threadIdx.x, i, j)) return;
-  update3d_zm_body<ODR, CZ>(in, ut, out, fl, ex, ey, ez, g, info->dtdx, info->dtdy, info->dtdz, ra, rb, i, j,
+  update3d_zm_body<ODR>(CZ ? CZ : cz, in, ut, out, fl, ex, ey, ez, g, info->dtdx, info->dtdy, info->dtdz, ra, rb, i, j,
                             b.plane);
 }
 
@@ -142,7 +143,22 @@ __global__ __launch_bounds__(256) void k_cfl3d(U3 u, G3 g, StepInfo *info, doubl
 }
 
 // ------------------------------------------------------------------- driver
-constexpr int kZChunk = 8;  // planes per thread of the z-marching edge/update kernels
+
+constexpr int kZChunk = 8;  // most planes per thread of the z-marching aux, edge and update kernels
+
+// Planes per thread: a longer march reads each plane of the z stencils once
+// more seldom, a shorter one makes more blocks.  At least 2048 blocks of 256 threads (two
+// wavefronts a SIMD) where the grid allows: with 8 planes everywhere the three
+// kernels of a 53x44x59 array took 81 us, with 1 they take 30; 72^3 8 steps
+// 5157 -> 4492 us (1), 104^3 12493 -> 12185 (2), 136^3 28621 -> 27787 (4); 264^3
+// update 1558 / 1500 / 1389 / 1330 us with 1 / 2 / 4 / 8, 1333 with 16.  8 is a
+// constant of its own kernels: as an argument it cost the 264^3 edges 3 %.
+static int zchunk(long cells)
+{
+  int cz = 1;
+  while (cz < kZChunk && cells >= 2L * cz * 256 * 2048) cz *= 2;
+  return cz;
+}
 
 static G3 geom3(Handle *h)
 {
@@ -201,12 +217,13 @@ static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double
   MLAU_LAUNCH(h, K_PRIM3D, (k_prim3d<ODR>), gflat, b256, in, P[0], P[1], P[2], P[3], P[4], P[5], P[6], P[7], g,
               h->bc);
   const bool zm = !(h->tune & 8);  // tune bit 3: plane-parallel aux/edge/update kernels instead of z-marching
-  const dim3 gz(plane_pieces(nx, ny) * ((nz + kZChunk - 1) / kZChunk));
+  const int cz = zchunk((long)nx * ny * nz);
+  const dim3 gz(plane_pieces(nx, ny) * ((nz + cz - 1) / cz));
   if (zm && h->s.ctw)
-    MLAU_LAUNCH(h, K_AUX3D, (k_aux3d_zm<1, kZChunk>), gz, b256, in, (const double *)P[0], (const double *)P[1],
+    MLAU_LAUNCH(h, K_AUX3D, (k_aux3d_zm<1>), gz, b256, cz, in, (const double *)P[0], (const double *)P[1],
                 (const double *)P[2], h->aux[0], h->aux[1], h->aux[2], h->aux[3], h->aux[4], h->aux[5], g, h->bc);
   else if (zm)
-    MLAU_LAUNCH(h, K_AUX3D, (k_aux3d_zm<0, kZChunk>), gz, b256, in, (const double *)P[0], (const double *)P[1],
+    MLAU_LAUNCH(h, K_AUX3D, (k_aux3d_zm<0>), gz, b256, cz, in, (const double *)P[0], (const double *)P[1],
                 (const double *)P[2], h->aux[0], h->aux[1], h->aux[2], h->aux[3], h->aux[4], h->aux[5], g, h->bc);
   else if (h->s.ctw)
     MLAU_LAUNCH(h, K_AUX3D, (k_aux3d<1>), gflat, b256, in, (const double *)P[0], (const double *)P[1],
@@ -233,9 +250,10 @@ static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double
   e.fzt = h->fz[4]; e.fzu = h->fz[5]; e.fcz0 = h->fcz[0]; e.fcz1 = h->fcz[1];
   e.ct0 = h->aux[0]; e.ct1 = h->aux[1]; e.ct2 = h->aux[2];
   e.ex = h->e[0]; e.ey = h->e[1]; e.ez = h->e[2];
-  if (zm)
-    MLAU_LAUNCH(h, K_EDGE3D, (k_edge3d_zm<ODR, kZChunk>), dim3(plane_pieces(nx, ny) * ((nz + kZChunk - 1) / kZChunk)),
-                b256, e, g);
+  if (zm && cz == kZChunk)
+    MLAU_LAUNCH(h, K_EDGE3D, (k_edge3d_zm<ODR, kZChunk>), gz, b256, cz, e, g);
+  else if (zm)
+    MLAU_LAUNCH(h, K_EDGE3D, (k_edge3d_zm<ODR, 0>), gz, b256, cz, e, g);
   else
     MLAU_LAUNCH(h, K_EDGE3D, (k_edge3d<ODR>), gcell, b256, e, g);
   Fl3 fl;
@@ -244,11 +262,12 @@ static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double
     fl.y[q] = h->fy[q];
     fl.z[q] = h->fz[q];
   }
-  if (zm)
-    MLAU_LAUNCH(h, K_UPD3D, (k_update3d_zm<ODR, kZChunk>),
-                dim3(plane_pieces(nx - 2 * g.xoff + 1, ny - 2 * g.yoff + 1) *
-                     ((nz - 2 * g.zoff + 1 + kZChunk - 1) / kZChunk)),
-                b256, in, ut, out, fl, (const double *)h->e[0], (const double *)h->e[1], (const double *)h->e[2], g,
+  const dim3 gu(plane_pieces(nx - 2 * g.xoff + 1, ny - 2 * g.yoff + 1) * ((nz - 2 * g.zoff + 1 + cz - 1) / cz));
+  if (zm && cz == kZChunk)
+    MLAU_LAUNCH(h, K_UPD3D, (k_update3d_zm<ODR, kZChunk>), gu, b256, cz, in, ut, out, fl, (const double *)h->e[0],
+                (const double *)h->e[1], (const double *)h->e[2], g, h->info, ra, rb, adv);
+  else if (zm)
+    MLAU_LAUNCH(h, K_UPD3D, (k_update3d_zm<ODR, 0>), gu, b256, cz, in, ut, out, fl, (const double *)h->e[0], (const double *)h->e[1], (const double *)h->e[2], g,
                 h->info, ra, rb, adv);
   else
     MLAU_LAUNCH(h, K_UPD3D, (k_update3d<ODR>),

@@ -142,17 +142,17 @@ __device__ __forceinline__ double ct_w4(double a0, double a1, double a2, double 
   return (vac + 0.5 * eps) / (vac + vbc + eps);
 }
 
-// aux3d_body on cells (i, j, kc*CZ ..): one thread walks CZ cells along z and
+// aux3d_body on cells (i, j, kc*cz ..): one thread walks cz cells along z and
 // keeps the values of the plane below that the CT weights and the z shock
 // sensor read (velocities and density at (i,j), (i-1,j), (i,j-1); Bx, By at
 // (i,j)), so that plane is not read again.  Same arithmetic as aux3d_body.
-template <int CTW, int CZ>
-__device__ __forceinline__ void aux3d_zm_body(U3 u, const double *vx, const double *vy, const double *vz, double *ct0,
+template <int CTW>
+__device__ __forceinline__ void aux3d_zm_body(int cz, U3 u, const double *vx, const double *vy, const double *vz, double *ct0,
                                               double *ct1, double *ct2, double *dvx, double *dvy, double *dvz, G3 g,
                                               const BcFlags &bc, int i, int j, int kc)
 {
   const long nx = g.nx, nxy = (long)g.nx * g.ny;
-  const int k0 = kc * CZ, k1 = (k0 + CZ - 1 < g.nz - 1) ? k0 + CZ - 1 : g.nz - 1;
+  const int k0 = kc * cz, k1 = (k0 + cz - 1 < g.nz - 1) ? k0 + cz - 1 : g.nz - 1;
   const bool hw = i >= 1, hs = j >= 1;
   const double *ro = u.f[0];
   // previous plane: (i,j): x,y,z,r; (i,j-1): y,z,r; (i-1,j): z,x,r; Bx, By at (i,j)
@@ -498,7 +498,7 @@ __host__ __device__ __forceinline__ unsigned plane_pieces(int nx, int ny) { retu
 
 // ------------------------------------------------------- z-marching variants
 // The same per-cell arithmetic as edge3d_body / update3d_body, but one thread
-// walks a chunk of CZ cells along z and keeps the z-stencil values of the
+// walks a chunk of cz cells along z and keeps the z-stencil values of the
 // previous cells in registers, so each plane of a z-differenced array is read
 // once per chunk instead of four to six times.
 
@@ -511,13 +511,13 @@ __device__ __forceinline__ double corner_sum_w(const double (&w)[6])
   return l + r;
 }
 
-// Column (i, j), planes kc*CZ.. kc*CZ+CZ-1 (any column of the grid).
-template <int ODR, int CZ>
-__device__ __forceinline__ void edge3d_zm_body(const Edge3 &e, G3 g, int i, int j, int kc)
+// Column (i, j), planes kc*cz.. kc*cz+cz-1 (any column of the grid).
+template <int ODR>
+__device__ __forceinline__ void edge3d_zm_body(int cz, const Edge3 &e, G3 g, int i, int j, int kc)
 {
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const long NX = nx, NXY = (long)nx * ny;
-  const int k0 = kc * CZ, k1 = (k0 + CZ - 1 < nz - 1) ? k0 + CZ - 1 : nz - 1;
+  const int k0 = kc * cz, k1 = (k0 + cz - 1 < nz - 1) ? k0 + cz - 1 : nz - 1;
   const bool ix = (i >= 3 && i <= nx - 3), jy = (j >= 3 && j <= ny - 3);
   double wxu[6], wcx[6], wyt[6], wcy[6];  // fxu, fcx1, fyt, fcy0 at planes k-3..k+2
   int kw = -10;                           // plane whose window is loaded
@@ -574,16 +574,16 @@ __device__ __forceinline__ void edge3d_zm_body(const Edge3 &e, G3 g, int i, int 
 }
 
 // Column (i, j) with xoff <= i <= nx-xoff, yoff <= j <= ny-yoff, planes
-// zoff+kc*CZ.. up to nz-zoff (one extra face per axis for the CT update).
-template <int ODR, int CZ>
-__device__ __forceinline__ void update3d_zm_body(U3 in, U3 ut, U3 out, const Fl3 &fl, const double *ex,
+// zoff+kc*cz.. up to nz-zoff (one extra face per axis for the CT update).
+template <int ODR>
+__device__ __forceinline__ void update3d_zm_body(int cz, U3 in, U3 ut, U3 out, const Fl3 &fl, const double *ex,
                                                  const double *ey, const double *ez, G3 g, double dtdx,
                                                  double dtdy, double dtdz, double ra, double rb, int i, int j, int kc)
 {
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const long NX = nx, NXY = (long)nx * ny;
-  const int k0 = g.zoff + kc * CZ;
-  const int k1 = (k0 + CZ - 1 < nz - g.zoff) ? k0 + CZ - 1 : nz - g.zoff;
+  const int k0 = g.zoff + kc * cz;
+  const int k1 = (k0 + cz - 1 < nz - g.zoff) ? k0 + cz - 1 : nz - g.zoff;
   const bool ci = i < nx - g.xoff, cj = j < ny - g.yoff;
   const int cz_[5] = {0, 2, 3, 1, 6};
   // windows over planes k-1..k+2: z fluxes of ro,mx,my,mz,en; ey (for Bx); ex (for By)

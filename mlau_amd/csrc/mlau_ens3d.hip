@@ -157,7 +157,7 @@ __global__ __launch_bounds__(256) void k_ens_aux3d(const EnsRec3D *__restrict__ 
     const unsigned np = plane_pieces(R.g.nx, R.g.ny);
     int i, j;
     if (!plane_cell(R.g, l_ % np, threadIdx.x, i, j)) continue;
-    aux3d_zm_body<CTW, kEnsZChunk>(sin ? R.u1 : R.u0, R.prim[0], R.prim[1], R.prim[2], R.aux[0], R.aux[1], R.aux[2],
+    aux3d_zm_body<CTW>(kEnsZChunk, sin ? R.u1 : R.u0, R.prim[0], R.prim[1], R.prim[2], R.aux[0], R.aux[1], R.aux[2],
                                    R.aux[3], R.aux[4], R.aux[5], R.g, R.bc, i, j, (int)(l_ / np));
   }
 }
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(256) void k_ens_edge3d(const EnsRec3D *__restrict__
     e.fzt = R.fl[2][4]; e.fzu = R.fl[2][5]; e.fcz0 = R.fc[2][0]; e.fcz1 = R.fc[2][1];
     e.ct0 = R.aux[0]; e.ct1 = R.aux[1]; e.ct2 = R.aux[2];
     e.ex = R.e[0]; e.ey = R.e[1]; e.ez = R.e[2];
-    edge3d_zm_body<ODR, kEnsZChunk>(e, R.g, i, j, kc);
+    edge3d_zm_body<ODR>(kEnsZChunk, e, R.g, i, j, kc);
   }
 }
 
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void k_ens_update3d(const EnsRec3D *__restrict
       fl.z[q] = R.fl[2][q];
     }
     const EnsState &S = st[e_.x];
-    update3d_zm_body<ODR, kEnsZChunk>(sin ? R.u1 : R.u0, R.u0, sout ? R.u1 : R.u0, fl, R.e[0], R.e[1], R.e[2], R.g,
+    update3d_zm_body<ODR>(kEnsZChunk, sin ? R.u1 : R.u0, R.u0, sout ? R.u1 : R.u0, fl, R.e[0], R.e[1], R.e[2], R.g,
                                       S.dtdx, S.dtdy, S.dtdz, ra, rb, i, j, kc);
   }
 }

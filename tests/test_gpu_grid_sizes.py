@@ -37,9 +37,11 @@ def test_2d_march_lengths(gpu, ny, nx, walls):
     s.close()
 
 
-@pytest.mark.parametrize("nz,ny,nx", [(4, 5, 6), (30, 21, 25), (63, 50, 70), (90, 101, 97)])
-def test_3d_march_lengths(gpu, nz, ny, nx):
-    """y- and z-sweep marches of 1 to 8 faces per lane, the last one cut short."""
+# y- and z-sweep marches of 1 to 8 faces per lane; 1, 2 and 4 planes per thread
+# in the aux, edge and update kernels; the last of each cut short
+@pytest.mark.parametrize("nz,ny,nx", [(4, 5, 6), (30, 21, 25), (7, 120, 125), (63, 50, 70), (85, 96, 97),
+                                      (131, 96, 127)])
+def test_3d_marches(gpu, nz, ny, nx):
     g, p = P.ot_vortex_3d(max(nx, ny, nz, 16))
     f0 = np.ascontiguousarray(g[:, :nz + 8, :ny + 8, :nx + 8])
     P.periodic_fill(f0)
