@@ -1,6 +1,9 @@
 // mlau_1d.hip -- 1D ideal-MHD step on gfx950 (FP64).
 //
-// One RK stage of 1D/SERIAL/shock/mhd_fd4c_1d.c:110-257 in two launches:
+// k_step1d runs one or more whole steps of 1D/SERIAL/shock/mhd_fd4c_1d.c:60-271 in
+// one launch (step1d_body): each block advances a window of cells with its own
+// halo, from u0 to u1 or back.  Very long grids, where the repeated halo cells
+// cost more than the launches, take a stage in two launches or one:
 //   k_sweep1d   primitives (:121-131, formed per stencil point) + reconstruction
 //               + Riemann solver, one wavefront per 63 faces (left face
 //               states passed by shuffle)                                :137-207
@@ -53,6 +56,28 @@ __global__ __launch_bounds__(256) void k_update1d(U1d in, U1d ut, U1d out, W1d w
   }
 }
 
+// K whole steps (step1d_body); block 0 advances the time.
+template <int ODR, int FLUX, int MIX, bool PER>
+__global__ __launch_bounds__(PER ? kWin1 : kWin1 + 64) void k_step1d(U1d in, U1d out, G1d g, StepInfo *info, int rk,
+                                                                     int K)
+{
+  __shared__ Lds1d S;
+  step1d_body<ODR, FLUX, MIX, PER>(in, out, g, info->dtdx, rk, K, blockIdx.x, threadIdx.x, S);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    for (int k = 0; k < K; k++) info->tim += info->dt;
+    info->nstep += K;
+  }
+}
+
+// blockIdx.y = field
+__global__ __launch_bounds__(256) void k_copy1d(U1d src, U1d dst, int nx)
+{
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= nx) return;
+#pragma unroll
+  for (int n = 0; n < 7; n++) dst.f[n][i] = src.f[n][i];
+}
+
 template <int ODR, int FLUX, int MIX, bool PER>
 __global__ __launch_bounds__(256) void k_stage1d(U1d in, U1d ut, U1d out, G1d g, StepInfo *info, double ra, double rb,
                                                  int copy_ghosts, int adv)
@@ -76,6 +101,12 @@ __global__ __launch_bounds__(256) void k_cfl1d(U1d u, G1d g, StepInfo *info, dou
   }
   v = block_max<256>(v);
   if (threadIdx.x == 0) cfl_finish(info, v, cfl, vfloor, dx, dx, dy, dz);
+}
+
+static void check1d(Handle *h, const U1d &u, const G1d &g, double cfl, double vfloor)
+{
+  MLAU_LAUNCH(h, K_CFL1D, k_cfl1d, dim3((g.nx + 255) / 256), dim3(256), u, g, h->info, cfl, vfloor, h->g.dx, h->g.dy,
+              h->g.dz);
 }
 
 static void views1d(Handle *h, U1d &u0, U1d &u1, W1d &w, G1d &g)
@@ -144,7 +175,51 @@ static void step1d(Handle *h)
   }
 }
 
+// Whole steps per launch: more save launches and repeat more cells at the
+// windows' edges.  Measured, us for 32 steps (MUSCL MLAU open / WCNS4 LHLLD periodic), a launch
+// or two per stage -> 1, 2, 4 steps per launch: 1024 cells 843 -> 558, 527, 534 /
+// 1049 -> 673, 625, 597; 65536: 1178 -> 854, 805, 784 / 1704 -> 1247, 1179, 1162;
+// 262144: 2292 -> 2019, 1899, 2193 / 3540 -> 3015, 2884, 3922; 1048576: 6461 -> 6885, 6936,
+// 8170 / 11050 -> 10566, 11347, 14478.  0: separate stage launches, also for
+// FP32 Riemann solvers and the mixed Roe solver, whose multiply-adds the
+// compiler would fuse otherwise here (rounding differences of 1e-9 to 1e-8).
+static int steps_per_launch1d(const Handle *h, bool cfl_mode)
+{
+  if ((h->tune & 8) || h->g.nx > 393216) return 0;
+  if (h->s.precision == MLAU_MIXED || (h->s.precision == MLAU_MIXED_RECON && h->s.flux == FLUX_ROE)) return 0;
+  if (cfl_mode) return 1;  // the next dt needs the whole grid
+  return h->g.nx > 131072 ? 2 : 4;
+}
+
+// Steps in launches of up to `most` whole steps, from one state to the other and
+// back; an odd number of launches ends with a copy into u0.
+template <int ODR, int FLUX, int MIX>
+static void steps1d(Handle *h, int nsteps, int most, bool cfl_mode, double cfl, double vfloor)
+{
+  U1d u0, u1;
+  W1d w;
+  G1d g;
+  views1d(h, u0, u1, w, g);
+  const int rk = h->s.rk, nx = g.nx;
+  const bool open = h->s.bc1d == MLAU_BC1D_OPEN;
+  int m = (nsteps + most - 1) / most;  // launches
+  if ((m & 1) && m < nsteps) m++;
+  for (int j = 0; j < m; j++) {
+    const int K = (int)((long)nsteps * (j + 1) / m - (long)nsteps * j / m);
+    const int own = kWin1 - 2 * win1_halo<ODR>(K, rk);
+    const dim3 gr((nx - 8 + own - 1) / own);
+    const U1d &in = j & 1 ? u1 : u0, &out = j & 1 ? u0 : u1;
+    if (open)
+      MLAU_LAUNCH(h, K_STEP1D, (k_step1d<ODR, FLUX, MIX, false>), gr, dim3(kWin1 + 64), in, out, g, h->info, rk, K);
+    else
+      MLAU_LAUNCH(h, K_STEP1D, (k_step1d<ODR, FLUX, MIX, true>), gr, dim3(kWin1), in, out, g, h->info, rk, K);
+    if (cfl_mode) check1d(h, out, g, cfl, vfloor);
+  }
+  if (m & 1) MLAU_LAUNCH(h, K_STEP1D, k_copy1d, dim3((nx + 255) / 256), dim3(256), u1, u0, nx);
+}
+
 typedef void (*Step1Fn)(Handle *);
+typedef void (*Steps1Fn)(Handle *, int, int, bool, double, double);
 template <int ODR, int MIX>
 static Step1Fn pick1f(int flux)
 {
@@ -165,20 +240,46 @@ static Step1Fn pick1(int flux, int precision)
   }
 }
 
+template <int ODR, int MIX>
+static Steps1Fn pick1sf(int flux)
+{
+  switch (flux) {
+  case FLUX_MLAU: return steps1d<ODR, FLUX_MLAU, MIX>;
+  case FLUX_ROE: return steps1d<ODR, FLUX_ROE, MLAU_FP64>;  // FP64 only (steps_per_launch1d)
+  case FLUX_HLLD: return steps1d<ODR, FLUX_HLLD, MIX>;
+  default: return steps1d<ODR, FLUX_LHLLD, MIX>;
+  }
+}
+template <int ODR>
+static Steps1Fn pick1s(int flux, int precision)
+{
+  return precision == MLAU_MIXED_RECON ? pick1sf<ODR, MLAU_MIXED_RECON>(flux) : pick1sf<ODR, MLAU_FP64>(flux);
+}
+
 int run_cfl_1d(Handle *h, double cfl, double vfloor)
 {
   U1d u0, u1;
   W1d w;
   G1d g;
   views1d(h, u0, u1, w, g);
-  MLAU_LAUNCH(h, K_CFL1D, k_cfl1d, dim3((g.nx + 255) / 256), dim3(256), u0, g, h->info, cfl, vfloor, h->g.dx, h->g.dy,
-              h->g.dz);
+  check1d(h, u0, g, cfl, vfloor);
   return (int)hipGetLastError();
 }
 
 int run_steps_1d(Handle *h, int nsteps, bool cfl_mode, double cfl, double vfloor)
 {
   if (h->g.xoff != 4) return (int)hipErrorInvalidValue;
+  if (const int most = steps_per_launch1d(h, cfl_mode)) {
+    Steps1Fn fs;
+    switch (h->s.odr) {
+    case 1: fs = pick1s<1>(h->s.flux, h->s.precision); break;
+    case 2: fs = pick1s<2>(h->s.flux, h->s.precision); break;
+    case 3: fs = pick1s<3>(h->s.flux, h->s.precision); break;
+    default: fs = pick1s<4>(h->s.flux, h->s.precision); break;
+    }
+    fs(h, nsteps, most, cfl_mode, cfl, vfloor);
+    return (int)hipGetLastError();
+  }
   Step1Fn fn;
   switch (h->s.odr) {
   case 1: fn = pick1<1>(h->s.flux, h->s.precision); break;

@@ -146,7 +146,58 @@ static __device__ void eigen_st_full(const double p[8], double gamma, double al[
   R[3][0] = 1.0;
 }
 
-// openbc1d_mhd with istt=0, iend=1 (1D/SERIAL/shock/openbc1d_mhd.c:21-175);
+// Characteristic open boundary of one side (openbc1d_mhd with istt=0, iend=1,
+// 1D/SERIAL/shock/openbc1d_mhd.c:21-175): the conserved values of the ghosts
+// from the primitives q[v][0] of the outermost interior cell and q[v][1] of the
+// ghost next to it (ro, vx, vy, vz, by, bz, pr).
+// SYNC: every thread of the wavefront passes one __syncthreads between the
+// eigensystem and the ghosts.
+template <bool SYNC>
+__device__ __forceinline__ void openbc1d_cell(const double (&q)[7][2], const G1d &g, double dtdx, unsigned side,
+                                              double (&vals)[7])
+{
+  const int sgn = side == 0 ? 1 : -1;
+  const double bx = g.bx, bx2 = bx * bx, gamma = g.gamma;
+  const double rob[2] = {q[0][0], q[0][1]}, vxb[2] = {q[1][0], q[1][1]}, vyb[2] = {q[2][0], q[2][1]};
+  const double vzb[2] = {q[3][0], q[3][1]}, bxb[2] = {bx, bx}, byb[2] = {q[4][0], q[4][1]};
+  const double bzb[2] = {q[5][0], q[5][1]}, prb[2] = {q[6][0], q[6][1]};
+  double p[8] = {0.5 * (rob[0] + rob[1]), 0.5 * (vxb[0] + vxb[1]), 0.5 * (vyb[0] + vyb[1]), 0.5 * (vzb[0] + vzb[1]),
+                 0.5 * (bxb[0] + bxb[1]), 0.5 * (byb[0] + byb[1]), 0.5 * (bzb[0] + bzb[1]), 0.5 * (prb[0] + prb[1])};
+  double al[7], L[7][7], R[7][7], w[7][2];
+  eigen_st_full(p, gamma, al, L, R);
+  if (SYNC) __syncthreads();
+  for (int j = 0; j < 2; j++)
+    for (int n = 0; n < 7; n++)
+      w[n][j] = (+L[n][0] * rob[j] + L[n][1] * vxb[j] + L[n][2] * vyb[j] + L[n][3] * vzb[j] + L[n][4] * byb[j] +
+                 L[n][5] * bzb[j] + L[n][6] * prb[j]);
+  for (int n = 0; n < 7; n++) {
+    const double sa = sgn * al[n];
+    w[n][1] = (sa > 0) ? w[n][1] : (1 + sa * dtdx) * w[n][1] - sa * dtdx * w[n][0];
+  }
+  double o[7];
+  for (int n = 0; n < 7; n++)
+    o[n] = R[0][n] * w[0][1] + R[1][n] * w[1][1] + R[2][n] * w[2][1] + R[3][n] * w[3][1] + R[4][n] * w[4][1] +
+           R[5][n] * w[5][1] + R[6][n] * w[6][1];
+  // o = (ro, vx, vy, vz, by, bz, pr) -> conservative
+  const double ro = o[0];
+  double mx = o[1], my = o[2], mz = o[3];
+  const double by = o[4], bz = o[5];
+  double en = o[6];
+  const double v2 = mx * mx + my * my + mz * mz;
+  const double b2 = bx2 + by * by + bz * bz;
+  en = en / (gamma - 1.0) + 0.5 * (ro * v2 + b2);
+  mx *= ro;
+  my *= ro;
+  mz *= ro;
+  vals[0] = ro;
+  vals[1] = mx;
+  vals[2] = my;
+  vals[3] = mz;
+  vals[4] = en;
+  vals[5] = by;
+  vals[6] = bz;
+}
+
 // thread 0 = left edge, thread 1 = right edge.  Reads the stage input and
 // writes the boundary ghosts of every buffer in `dst` (the stage output and
 // the step-start state, so later stages and the final state both see them).
@@ -157,51 +208,27 @@ __device__ __forceinline__ void openbc1d_body(U1d in, U1d dst0, U1d dst1, G1d g,
   const int sgn = side == 0 ? 1 : -1;
   const int si = side == 0 ? xoff : nx - xoff - 1;
   const int so = si - sgn;
-  const double bx = g.bx, bx2 = bx * bx, gamma = g.gamma;
-  double rob[2], vxb[2], vyb[2], vzb[2], bxb[2], byb[2], bzb[2], prb[2];
+  const double bx = g.bx, gamma = g.gamma;
+  double q[7][2];
   const int idx[2] = {si, so};
   for (int j = 0; j < 2; j++) {
     const int ss = idx[j];
-    rob[j] = in.f[0][ss];
-    const double iro = 1.0 / rob[j];
-    vxb[j] = in.f[1][ss] * iro;
-    vyb[j] = in.f[2][ss] * iro;
-    vzb[j] = in.f[3][ss] * iro;
-    bxb[j] = bx;
-    byb[j] = in.f[5][ss];
-    bzb[j] = in.f[6][ss];
-    const double v2 = vxb[j] * vxb[j] + vyb[j] * vyb[j] + vzb[j] * vzb[j];
-    const double b2 = bxb[j] * bxb[j] + byb[j] * byb[j] + bzb[j] * bzb[j];
-    prb[j] = (gamma - 1.0) * (in.f[4][ss] - 0.5 * (rob[j] * v2 + b2));
+    const double ro = in.f[0][ss];
+    const double iro = 1.0 / ro;
+    const double vx = in.f[1][ss] * iro, vy = in.f[2][ss] * iro, vz = in.f[3][ss] * iro;
+    const double by = in.f[5][ss], bz = in.f[6][ss];
+    const double v2 = vx * vx + vy * vy + vz * vz;
+    const double b2 = bx * bx + by * by + bz * bz;
+    q[0][j] = ro;
+    q[1][j] = vx;
+    q[2][j] = vy;
+    q[3][j] = vz;
+    q[4][j] = by;
+    q[5][j] = bz;
+    q[6][j] = (gamma - 1.0) * (in.f[4][ss] - 0.5 * (ro * v2 + b2));
   }
-  double p[8] = {0.5 * (rob[0] + rob[1]), 0.5 * (vxb[0] + vxb[1]), 0.5 * (vyb[0] + vyb[1]), 0.5 * (vzb[0] + vzb[1]),
-                 0.5 * (bxb[0] + bxb[1]), 0.5 * (byb[0] + byb[1]), 0.5 * (bzb[0] + bzb[1]), 0.5 * (prb[0] + prb[1])};
-  double al[7], L[7][7], R[7][7], w[7][2];
-  eigen_st_full(p, gamma, al, L, R);
-  for (int j = 0; j < 2; j++)
-    for (int n = 0; n < 7; n++)
-      w[n][j] = (+L[n][0] * rob[j] + L[n][1] * vxb[j] + L[n][2] * vyb[j] + L[n][3] * vzb[j] + L[n][4] * byb[j] +
-                 L[n][5] * bzb[j] + L[n][6] * prb[j]);
-  for (int n = 0; n < 7; n++) {
-    const double sa = sgn * al[n];
-    w[n][1] = (sa > 0) ? w[n][1] : (1 + sa * dtdx) * w[n][1] - sa * dtdx * w[n][0];
-  }
-  double q[7];
-  for (int n = 0; n < 7; n++)
-    q[n] = R[0][n] * w[0][1] + R[1][n] * w[1][1] + R[2][n] * w[2][1] + R[3][n] * w[3][1] + R[4][n] * w[4][1] +
-           R[5][n] * w[5][1] + R[6][n] * w[6][1];
-  // q = (ro, vx, vy, vz, by, bz, pr) -> conservative
-  const double ro = q[0];
-  double mx = q[1], my = q[2], mz = q[3];
-  const double by = q[4], bz = q[5];
-  double en = q[6];
-  const double v2 = mx * mx + my * my + mz * mz;
-  const double b2 = bx2 + by * by + bz * bz;
-  en = en / (gamma - 1.0) + 0.5 * (ro * v2 + b2);
-  mx *= ro;
-  my *= ro;
-  mz *= ro;
-  const double vals[7] = {ro, mx, my, mz, en, by, bz};
+  double vals[7];
+  openbc1d_cell<false>(q, g, dtdx, side, vals);
   U1d *dsts[2] = {&dst0, &dst1};
   for (int d = 0; d < 2; d++) {
     for (int n = 0; n < 7; n++) {
@@ -309,6 +336,246 @@ __device__ __forceinline__ void stage1d_body(U1d in, U1d ut, U1d out, G1d g, dou
       if (c >= nx - 2 * xoff && c < nx - xoff) out.f[n][c - (nx - 2 * xoff)] = v;  // f[j] = f[nx-2xoff+j]
       if (c >= xoff && c < 2 * xoff) out.f[n][nx - 2 * xoff + c] = v;              // f[nx-1-j] = f[2xoff-1-j]
     }
+  }
+}
+
+// ------------------------------------------------------------- whole steps
+// K steps in one launch.  A block holds a window of kWin1 cells, one per lane
+// of its first four wavefronts, with the state in registers; primitives, left
+// states and fluxes pass between lanes through LDS.  Nothing crosses blocks:
+// each stage the outer cells of the window lose their meaning by the reach of
+// its stencils (kReach), so a window of kWin1 gives win1_cells(K, rk) cells after K
+// steps, and neighbouring blocks form the rest for themselves.  On a periodic
+// grid the window wraps around (ghosts are copies); at an open end the ghosts are cells of the
+// window, and a fifth wavefront forms their new values during the first
+// stage's sweep (it reads the same stage input).
+//
+// What bounds a 1D grid is the chain of one cell's stage (about 4 us) and,
+// with a launch per stage, the launches: 1024 cells took 26 us a step in four
+// launches at ODR 2, and 8191 cells 34 us in six at ODR 4.
+constexpr int kWin1 = 256;
+template <int ODR>
+constexpr int kReach = ODR <= 2 ? 3 : 4;  // faces i..i+1 or i-1..i+2, each from the cells 3 below to 2 above
+template <int ODR>
+__host__ __device__ __forceinline__ int win1_halo(int K, int rk)
+{
+  const int h = K * rk * kReach<ODR>;
+  return h < 4 ? 4 : h;  // an end's ghosts lie in the window of the block that writes them
+}
+
+struct Lds1d {
+  double q[7][kWin1];  // primitives ro, vx, vy, vz, by, bz, pr
+  double m[kWin1];     // squared Mach number
+  double l[7][kWin1];  // left state of the face above each cell
+  double f[7][kWin1];  // flux through the face below each cell, argument order
+  double end[2][7];    // new ghosts of the open ends
+};
+
+// Flux differences of cell a (4 <= a <= nx-5) straight from the arrays, ghosts as
+// they stand: what a stage of the separate kernels gives.
+template <int ODR, int FLUX, int MIX>
+__device__ __forceinline__ void flux_diff1d(const U1d &in, const G1d &g, int a, double (&du)[7])
+{
+  constexpr int lo = ODR <= 2 ? 0 : -1, hi = ODR <= 2 ? 1 : 2;  // faces a+lo..a+hi
+  const double bx2 = g.bx * g.bx;
+  double F[4][7], L[7];
+#pragma unroll 1
+  for (int j = a + lo - 1; j <= a + hi; j++) {
+    Stencil W;
+    double r[5];
+#pragma unroll
+    for (int m = 0; m < 5; m++) {
+      const int q = j - 2 + m;
+      const double ro = in.f[0][q], iro = 1.0 / ro;
+      const double vx = in.f[1][q] * iro, vy = in.f[2][q] * iro, vz = in.f[3][q] * iro;
+      const double by = in.f[5][q], bz = in.f[6][q];
+      const double v2 = vx * vx + vy * vy + vz * vz;
+      const double b2 = bx2 + by * by + bz * bz;
+      const double pr = (g.gamma - 1.0) * (in.f[4][q] - 0.5 * (ro * v2 + b2));
+      const double cs2 = g.gamma * pr / ro;
+      r[m] = v2 / cs2;
+      W.q[0][m] = ro;
+      W.q[1][m] = vx;
+      W.q[2][m] = vy;
+      W.q[3][m] = vz;
+      W.q[4][m] = by;
+      W.q[5][m] = bz;
+      W.q[6][m] = pr;
+    }
+    const bool sup = dmax(r[1], dmax(r[2], r[3])) >= 1.0;
+    double vl[7], vr[7], f[7];
+    recon_p<ODR, MIX>(W, sup, g.bx, g.gamma, vl, vr);
+    if (j >= a + lo) {
+      riemann_p<FLUX, MIX>(L, vr, g.bx, g.gamma, W.q[1][2] - W.q[1][1], 0.0, f);
+      const double fa[7] = {f[0], f[1], f[2], f[3], f[6], f[4], f[5]};
+#pragma unroll
+      for (int n = 0; n < 7; n++) {
+        F[0][n] = F[1][n];
+        F[1][n] = F[2][n];
+        F[2][n] = F[3][n];
+        F[3][n] = fa[n];
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < 7; n++) L[n] = vl[n];
+  }
+#pragma unroll
+  for (int n = 0; n < 7; n++)
+    du[n] = ODR <= 2 ? diff4<ODR>(0.0, F[2][n], F[3][n], 0.0) : diff4<ODR>(F[0][n], F[1][n], F[2][n], F[3][n]);
+}
+
+template <int ODR, int FLUX, int MIX, bool PER>
+__device__ __forceinline__ void step1d_body(const U1d &in, const U1d &out, const G1d &g, double dtdx, int rk, int K,
+                                            unsigned b, unsigned tid, Lds1d &S)
+{
+  const int nx = g.nx, N = nx - 8, H = win1_halo<ODR>(K, rk), own = kWin1 - 2 * H;
+  const int first = 4 + (int)b * own;        // first cell this block writes
+  const int last = first + own < nx - 4 ? first + own : nx - 4;
+  const int t = (int)tid, c0 = first - H;    // lane t holds cell c0 + t
+  const int c = c0 + t;
+  const bool cell = tid < kWin1;
+  // lanes outside the grid hold copies that no cell in reach of the result reads
+  const int at = PER ? 4 + (((c - 4) % N) + N) % N : (c < 0 ? 0 : (c > nx - 1 ? nx - 1 : c));
+  const bool inner = PER || (c >= 4 && c <= nx - 5);
+  const bool end0 = !PER && c0 <= 3, end1 = !PER && c0 + kWin1 - 1 >= nx - 4;
+  double u[7], ut[7];
+  if (cell) {
+#pragma unroll
+    for (int n = 0; n < 7; n++) u[n] = in.f[n][at];
+  }
+  // A periodic window that wraps takes the cells beyond an end from the other
+  // end; ghosts that the caller has filled otherwise count for the first stage.
+  bool raw = false;
+  if (PER && (c0 < 4 || c0 + kWin1 > nx - 4)) {
+    int differ = 0;
+    if (tid < 8) {
+#pragma unroll
+      for (int n = 0; n < 7; n++)
+        differ |= __double_as_longlong(in.f[n][tid]) != __double_as_longlong(in.f[n][nx - 8 + tid]);
+    }
+    raw = __syncthreads_or(differ) != 0;
+  }
+  const double bx2 = g.bx * g.bx;
+  const double ra1 = 0.5 + (rk - 2) * 0.25, rb1 = 0.5 - (rk - 2) * 0.25;
+  for (int s = 0; s < K * rk; s++) {
+    const int st = s % rk;
+    if (cell) {
+      if (st == 0) {
+#pragma unroll
+        for (int n = 0; n < 7; n++) ut[n] = u[n];
+      }
+    }
+    if (PER && raw && s == 0) {
+      double du[7];
+      flux_diff1d<ODR, FLUX, MIX>(in, g, at, du);
+#pragma unroll
+      for (int n = 0; n < 7; n++) u[n] = 0.0 * ut[n] + 1.0 * (u[n] - dtdx * du[n]);
+      continue;
+    }
+    if (cell) {
+      const double iro = 1.0 / u[0];
+      const double vx = u[1] * iro, vy = u[2] * iro, vz = u[3] * iro;
+      const double v2 = vx * vx + vy * vy + vz * vz;
+      const double b2 = bx2 + u[5] * u[5] + u[6] * u[6];
+      const double pr = (g.gamma - 1.0) * (u[4] - 0.5 * (u[0] * v2 + b2));
+      S.q[0][t] = u[0];
+      S.q[1][t] = vx;
+      S.q[2][t] = vy;
+      S.q[3][t] = vz;
+      S.q[4][t] = u[5];
+      S.q[5][t] = u[6];
+      S.q[6][t] = pr;
+      const double cs2 = g.gamma * pr / u[0];  // supersonic switch (mhd_fd4c_1d.c:155-166)
+      S.m[t] = v2 / cs2;
+    }
+    __syncthreads();
+    double vr[7], dv0 = 0.0;
+    if (cell) {
+      Stencil W;
+#pragma unroll
+      for (int m = 0; m < 5; m++) {
+        int p = t + m - 2;
+        p = p < 0 ? 0 : (p > kWin1 - 1 ? kWin1 - 1 : p);
+#pragma unroll
+        for (int v = 0; v < 7; v++) W.q[v][m] = S.q[v][p];
+      }
+      const int lo = t > 0 ? t - 1 : 0, hi = t < kWin1 - 1 ? t + 1 : kWin1 - 1;
+      const bool sup = dmax(S.m[lo], dmax(S.m[t], S.m[hi])) >= 1.0;
+      double vl[7];
+      recon_p<ODR, MIX>(W, sup, g.bx, g.gamma, vl, vr);
+      dv0 = W.q[1][2] - W.q[1][1];
+#pragma unroll
+      for (int k = 0; k < 7; k++) S.l[k][t] = vl[k];
+    } else if (!PER && st == 0 && (end0 || end1)) {
+      // open ends: the even lanes form the left one's ghosts, the odd lanes the
+      // right one's (of clamped cells where the window does not reach it), the
+      // first half beside the sweep and the second beside the Riemann solver
+      const unsigned side = tid & 1;
+      int ti = (side == 0 ? 4 : nx - 5) - c0, to = (side == 0 ? 3 : nx - 4) - c0;
+      ti = ti < 0 ? 0 : (ti > kWin1 - 1 ? kWin1 - 1 : ti);
+      to = to < 0 ? 0 : (to > kWin1 - 1 ? kWin1 - 1 : to);
+      double q[7][2];
+#pragma unroll
+      for (int v = 0; v < 7; v++) {
+        q[v][0] = S.q[v][ti];
+        q[v][1] = S.q[v][to];
+      }
+      double vals[7];
+      openbc1d_cell<true>(q, g, dtdx, side, vals);
+      if (tid < kWin1 + 2) {
+#pragma unroll
+        for (int n = 0; n < 7; n++) S.end[side][n] = vals[n];
+      }
+      __syncthreads();
+      continue;
+    }
+    __syncthreads();
+    if (cell) {
+      double L[7], f[7];
+      const int lo = t > 0 ? t - 1 : 0;
+#pragma unroll
+      for (int k = 0; k < 7; k++) L[k] = S.l[k][lo];
+      riemann_p<FLUX, MIX>(L, vr, g.bx, g.gamma, dv0, 0.0, f);
+      S.f[0][t] = f[0];
+      S.f[1][t] = f[1];
+      S.f[2][t] = f[2];
+      S.f[3][t] = f[3];
+      S.f[4][t] = f[6];
+      S.f[5][t] = f[4];
+      S.f[6][t] = f[5];
+    }
+    __syncthreads();  // the fifth wavefront's third, too, where it has formed ghosts
+    if (cell) {
+      if (inner) {
+        const double ra = st == 0 ? 0.0 : (st == 1 ? ra1 : 1. / 3.), rb = st == 0 ? 1.0 : (st == 1 ? rb1 : 2. / 3.);
+        const int p0 = t > 0 ? t - 1 : 0, p2 = t < kWin1 - 1 ? t + 1 : t, p3 = t < kWin1 - 2 ? t + 2 : p2;
+#pragma unroll
+        for (int n = 0; n < 7; n++) {
+          const double du = diff4<ODR>(ODR <= 2 ? 0.0 : S.f[n][p0], S.f[n][t], S.f[n][p2], ODR <= 2 ? 0.0 : S.f[n][p3]);
+          u[n] = ra * ut[n] + rb * (u[n] - dtdx * du);
+        }
+      } else if (st == 0) {
+        const int side = c < 4 ? 0 : 1;
+        if (side ? end1 : end0) {
+#pragma unroll
+          for (int n = 0; n < 7; n++) u[n] = S.end[side][n];
+        }
+      }
+    }
+  }
+  if (!cell) return;
+  if (c >= first && c < last) {
+#pragma unroll
+    for (int n = 0; n < 7; n++) {
+      out.f[n][c] = u[n];
+      if (PER) {
+        if (c >= nx - 8 && c < nx - 4) out.f[n][c - (nx - 8)] = u[n];  // f[j] = f[nx-2xoff+j]
+        if (c >= 4 && c < 8) out.f[n][nx - 8 + c] = u[n];              // f[nx-1-j] = f[2xoff-1-j]
+      }
+    }
+  } else if (!PER && ((c >= 0 && c < 4 && first == 4) || (c > nx - 5 && c < nx && last == nx - 4))) {
+#pragma unroll
+    for (int n = 0; n < 7; n++) out.f[n][c] = u[n];
   }
 }
 

@@ -53,3 +53,50 @@ def test_3d_marches(gpu, nz, ny, nx):
     s.step(1)
     assert_same(s.download(), f_o, "3D %dx%dx%d" % (nx, ny, nz))
     s.close()
+
+
+# whole steps per launch in 1D: windows of 256 cells that own 256 - 2*halo, so
+# one, two and more windows, a last one of a single cell, grids smaller than the
+# halo, odd and even launch counts, and each number of steps per launch
+@pytest.mark.parametrize("bc", ["open", "periodic", "periodic, other ghosts"])
+@pytest.mark.parametrize("n,odr,rk,flux,steps", [
+    (4, 2, 3, "mlau", 3), (5, 4, 3, "lhlld", 2), (9, 1, 1, "hlld", 1), (160, 4, 3, "lhlld", 8),
+    (161, 4, 3, "mlau", 9), (184, 2, 3, "mlau", 12), (369, 2, 3, "lhlld", 7), (238, 2, 3, "roe", 1),
+    (239, 3, 2, "hlld", 5), (500, 4, 1, "lhlld", 6), (140001, 2, 3, "mlau", 3), (400003, 4, 3, "lhlld", 1)])
+def test_1d_windows(gpu, bc, n, odr, rk, flux, steps):
+    f0, p = P.brio_wu(max(n, 16))
+    f0 = np.ascontiguousarray(f0[:, (max(n, 16) - n) // 2:][:, :n + 8])
+    x = np.arange(n + 8) / n
+    f0[2] += 0.1 * f0[0] * np.sin(7 * x)
+    f0[4] += 0.5 * f0[2] ** 2 / f0[0]
+    if bc == "periodic":
+        f0[:, :4], f0[:, -4:] = f0[:, n:n + 4].copy(), f0[:, 4:8].copy()
+    dt = 0.2 / n / 4.0
+    f_o = f0.copy()
+    for _ in range(steps):
+        O.step_1d(f_o, p["bx"], dt, 1.0 / n, 4, p["gamma"], O.scheme(odr, rk, flux, 1), periodic=bc != "open")
+    s = M.Solver(f0, M.scheme(odr, rk, flux, 1, bc1d=bc.split(",")[0]), 1.0 / n, gamma=p["gamma"], bx=p["bx"])
+    s.set_dt(dt)
+    s.step(steps)
+    assert_same(s.download(), f_o, "1D %s n=%d" % (bc, n))
+    t, _, k = s.time()
+    assert k == steps and abs(t - steps * dt) < 1e-12
+    s.close()
+
+
+@pytest.mark.parametrize("bc", ["open", "periodic"])
+@pytest.mark.parametrize("steps", [1, 2, 9])
+def test_1d_cfl_loop(gpu, bc, steps):
+    """dt from the whole grid after every step: one step per launch."""
+    f0, p = P.brio_wu(301)
+    f_o = f0.copy()
+    dt = 0.4 * p["dx"] / O.vmax_1d(f_o, p["bx"], p["gamma"])
+    for _ in range(steps):
+        O.step_1d(f_o, p["bx"], dt, p["dx"], 4, p["gamma"], O.scheme(2, 3, "mlau", 1), periodic=bc != "open")
+        dt = 0.4 * p["dx"] / O.vmax_1d(f_o, p["bx"], p["gamma"])
+    s = M.Solver(f0, M.scheme(2, 3, "mlau", 1, bc1d=bc), p["dx"], gamma=p["gamma"], bx=p["bx"])
+    s.cfl(0.4, 1.0)
+    s.step_cfl(steps, 0.4, 1.0)
+    assert s.time()[1] == dt
+    assert_same(s.download(), f_o, "1D cfl loop " + bc)
+    s.close()
