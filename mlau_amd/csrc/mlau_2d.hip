@@ -182,7 +182,7 @@ static void sweeps2d(Handle *h, const U2 &in, const W2 &w, const G2 &g)
   sd.fork(1);
   MLAU_LAUNCH(h, K_XSWEEP2D, (k_xsweep2d<ODR, FLUX, MIX>), gx, dim3(256), in, w, g);
   sd.enter(0);
-  const int ch = ychunk(h, g);
+  const int ch = whole_march<FLUX, MIX> ? kMarch : ychunk(h, g);
   const dim3 gy((g.nx + 63) / 64, (g.ny - 5 + ch - 1) / ch);
   if (split_march<MIX>(ch))
     MLAU_LAUNCH(h, K_YSWEEP2D, (k_ysweep2d<ODR, FLUX, MIX, MIX != MLAU_FP64>), gy, dim3(64), in, w, g, ch);

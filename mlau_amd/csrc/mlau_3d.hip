@@ -232,8 +232,9 @@ static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double
     MLAU_LAUNCH(h, K_AUX3D, (k_aux3d<0>), gflat, b256, in, (const double *)P[0], (const double *)P[1],
                 (const double *)P[2], h->aux[0], h->aux[1], h->aux[2], h->aux[3], h->aux[4], h->aux[5], g, h->bc);
   const long xw = xsweep_waves((long)ny * nz, nx), yw = ((long)nx * nz + 63) / 64, zw = ((long)nx * ny + 63) / 64;
-  const int chy = march_chunk(yw, ny - 5, xw + zw * nz, 0.2, kMarch, MIX != MLAU_FP64);
-  const int chz = march_chunk(zw, nz - 5, xw + yw * ny, 0.2, kMarch, MIX != MLAU_FP64);
+  const bool whole = whole_march<FLUX, MIX>;
+  const int chy = whole ? kMarch : march_chunk(yw, ny - 5, xw + zw * nz, 0.2, kMarch, MIX != MLAU_FP64);
+  const int chz = whole ? kMarch : march_chunk(zw, nz - 5, xw + yw * ny, 0.2, kMarch, MIX != MLAU_FP64);
   Side sd(h);  // the y and z sweeps beside the x sweep
   sd.fork(2);
   MLAU_LAUNCH(h, K_XSWEEP3D, (k_xsweep3d<ODR, FLUX, MIX>), dim3((unsigned)((xw + 3) / 4)), b256,
