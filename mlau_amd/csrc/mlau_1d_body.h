@@ -40,7 +40,7 @@ __device__ __forceinline__ void sweep1d_body(U1d u, W1d w, G1d g, unsigned bx, u
   for (int m = 0; m < 5; m++) {
     const int q = cc - 2 + m;
     const double ro = u.f[0][q];
-    const double iro = 1.0 / ro;
+    const double iro = rcp_ieee(ro);
     const double vx = u.f[1][q] * iro, vy = u.f[2][q] * iro, vz = u.f[3][q] * iro;
     const double by = u.f[5][q], bz = u.f[6][q];
     const double v2 = vx * vx + vy * vy + vz * vz;
@@ -286,7 +286,7 @@ __device__ __forceinline__ void stage1d_body(U1d in, U1d ut, U1d out, G1d g, dou
   for (int m = 0; m < 5; m++) {
     const int q = cc - 2 + m;
     const double ro = in.f[0][q];
-    const double iro = 1.0 / ro;
+    const double iro = rcp_ieee(ro);
     const double vx = in.f[1][q] * iro, vy = in.f[2][q] * iro, vz = in.f[3][q] * iro;
     const double by = in.f[5][q], bz = in.f[6][q];
     const double v2 = vx * vx + vy * vy + vz * vz;
@@ -365,7 +365,7 @@ __host__ __device__ __forceinline__ int win1_halo(int K, int rk)
 
 struct Lds1d {
   double q[7][kWin1];  // primitives ro, vx, vy, vz, by, bz, pr
-  double m[kWin1];     // squared Mach number
+  int m[kWin1];        // supersonic
   double l[7][kWin1];  // left state of the face above each cell
   double f[7][kWin1];  // flux through the face below each cell, argument order
   double end[2][7];    // new ghosts of the open ends
@@ -473,7 +473,7 @@ __device__ __forceinline__ void step1d_body(const U1d &in, const U1d &out, const
       continue;
     }
     if (cell) {
-      const double iro = 1.0 / u[0];
+      const double iro = rcp_ieee(u[0]);
       const double vx = u[1] * iro, vy = u[2] * iro, vz = u[3] * iro;
       const double v2 = vx * vx + vy * vy + vz * vz;
       const double b2 = bx2 + u[5] * u[5] + u[6] * u[6];
@@ -485,8 +485,7 @@ __device__ __forceinline__ void step1d_body(const U1d &in, const U1d &out, const
       S.q[4][t] = u[5];
       S.q[5][t] = u[6];
       S.q[6][t] = pr;
-      const double cs2 = g.gamma * pr / u[0];  // supersonic switch (mhd_fd4c_1d.c:155-166)
-      S.m[t] = v2 / cs2;
+      S.m[t] = ratio_ge1(v2, quot_ieee(g.gamma * pr, u[0]));  // supersonic switch (mhd_fd4c_1d.c:155-166)
     }
     __syncthreads();
     double vr[7], dv0 = 0.0;
@@ -500,7 +499,7 @@ __device__ __forceinline__ void step1d_body(const U1d &in, const U1d &out, const
         for (int v = 0; v < 7; v++) W.q[v][m] = S.q[v][p];
       }
       const int lo = t > 0 ? t - 1 : 0, hi = t < kWin1 - 1 ? t + 1 : kWin1 - 1;
-      const bool sup = dmax(S.m[lo], dmax(S.m[t], S.m[hi])) >= 1.0;
+      const bool sup = S.m[lo] | S.m[t] | S.m[hi];
       double vl[7];
       recon_p<ODR, MIX>(W, sup, g.bx, g.gamma, vl, vr);
       dv0 = W.q[1][2] - W.q[1][1];

@@ -73,7 +73,7 @@ __device__ __forceinline__ Prim2 prim2d_point(const U2 &u, const G2 &g, const Bc
     P.cy = sg * bc_centre<ODR>(by[-nx], by[0], by[nx], by[2 * nx]);
   }
   P.ro = u.f[0][s];
-  P.iro = 1.0 / P.ro;
+  P.iro = rcp_ieee(P.ro);
   P.vx = u.f[1][s] * P.iro;
   P.vy = u.f[2][s] * P.iro;
   P.vz = u.f[3][s] * P.iro;
@@ -88,6 +88,10 @@ __device__ __forceinline__ double prim2d_pr(const U2 &u, const G2 &g, const Prim
   return (g.gamma - 1.0) * (u.f[4][s] - 0.5 * (P.ro * P.v2 + b2));
 }
 __device__ __forceinline__ double prim2d_m2(const G2 &g, const Prim2 &P) { return P.v2 / (g.gamma * P.pr * P.iro); }
+__device__ __forceinline__ bool prim2d_sup(const G2 &g, const Prim2 &P)  // prim2d_m2 >= 1
+{
+  return ratio_ge1(P.v2, g.gamma * P.pr * P.iro);
+}
 
 // Any cell (i, j) of the grid.
 template <int ODR>
@@ -114,9 +118,9 @@ __device__ __forceinline__ double dvx2d_point(const U2 &u, const G2 &g, const Bc
   const int si = bc_src(i, g.nx, g.xoff, 0, -bc.dnx[1], &sg);
   const int sj = bc_src(j, g.ny, g.yoff, 0, +bc.dny[1], &sg);
   const long q = (long)sj * g.nx + si;
-  const double vm = u.f[1][q - 1] * (1.0 / u.f[0][q - 1]);
-  const double v0 = u.f[1][q] * (1.0 / u.f[0][q]);
-  const double vp = u.f[1][q + 1] * (1.0 / u.f[0][q + 1]);
+  const double vm = u.f[1][q - 1] * rcp_ieee(u.f[0][q - 1]);
+  const double v0 = u.f[1][q] * rcp_ieee(u.f[0][q]);
+  const double vp = u.f[1][q + 1] * rcp_ieee(u.f[0][q + 1]);
   return sg * dmin((vp - v0), (v0 - vm));
 }
 __device__ __forceinline__ double dvy2d_point(const U2 &u, const G2 &g, const BcFlags &bc, int i, int j)
@@ -125,9 +129,9 @@ __device__ __forceinline__ double dvy2d_point(const U2 &u, const G2 &g, const Bc
   const int si = bc_src(i, g.nx, g.xoff, 0, +bc.dnx[2], &sg);
   const int sj = bc_src(j, g.ny, g.yoff, 0, -bc.dny[2], &sg);
   const long q = (long)sj * g.nx + si, N = g.nx;
-  const double vm = u.f[2][q - N] * (1.0 / u.f[0][q - N]);
-  const double v0 = u.f[2][q] * (1.0 / u.f[0][q]);
-  const double vp = u.f[2][q + N] * (1.0 / u.f[0][q + N]);
+  const double vm = u.f[2][q - N] * rcp_ieee(u.f[0][q - N]);
+  const double v0 = u.f[2][q] * rcp_ieee(u.f[0][q]);
+  const double vp = u.f[2][q + N] * rcp_ieee(u.f[0][q + N]);
   return sg * dmin((vp - v0), (v0 - vm));
 }
 
@@ -144,13 +148,13 @@ __device__ __forceinline__ void aux2d_body(U2 u, W2 w, G2 g, BcFlags bc, int i, 
     double vxc = 0.25 * (w.vx[a - 1] + w.vx[a] + w.vx[c - 1] + w.vx[c]);
     double vyc = 0.25 * (w.vy[a - 1] + w.vy[a] + w.vy[c - 1] + w.vy[c]);
     double roc = 0.25 * (u.f[0][a - 1] + u.f[0][a] + u.f[0][c - 1] + u.f[0][c]);
-    roc = 1.0 / sqrt(roc);
+    roc = rcp_ieee(sqrt_ieee(roc));
     const double bxc = 0.5 * (u.f[5][a] + u.f[5][c]);
     const double byc = 0.5 * (u.f[6][c - 1] + u.f[6][c]);
     vxc = fabs(vxc) + fabs(bxc * roc);
     vyc = fabs(vyc) + fabs(byc * roc);
     const double eps = 1e-6;
-    ctx = (vxc + 0.5 * eps) / (vxc + vyc + eps);
+    ctx = quot_ieee(vxc + 0.5 * eps, vxc + vyc + eps);
   }
   w.ctx[s] = ctx;
   double sg = 1.0;
@@ -172,7 +176,7 @@ __device__ __forceinline__ void aux2d_body(U2 u, W2 w, G2 g, BcFlags bc, int i, 
 // bits the two kernels give; the primitive arrays are not read back.
 __device__ __forceinline__ double vel2d(const U2 &u, long q, int comp)
 {
-  const double iro = 1.0 / u.f[0][q];
+  const double iro = rcp_ieee(u.f[0][q]);
   return u.f[comp][q] * iro;
 }
 
@@ -192,7 +196,7 @@ __device__ __forceinline__ void primaux2d_body(U2 u, W2 w, G2 g, const BcFlags &
   const double *byp = u.f[6] + (long)sj * nx + si;
   const double cy = sg * bc_centre<ODR>(byp[-nx], byp[0], byp[nx], byp[2 * nx]);
   const double ro = u.f[0][s];
-  const double iro = 1.0 / ro;
+  const double iro = rcp_ieee(ro);
   const double vx = u.f[1][s] * iro;
   const double vy = u.f[2][s] * iro;
   const double vz = u.f[3][s] * iro;
@@ -214,13 +218,13 @@ __device__ __forceinline__ void primaux2d_body(U2 u, W2 w, G2 g, const BcFlags &
     double vxc = 0.25 * (vel2d(u, a - 1, 1) + vel2d(u, a, 1) + vel2d(u, c - 1, 1) + vx);
     double vyc = 0.25 * (vel2d(u, a - 1, 2) + vel2d(u, a, 2) + vel2d(u, c - 1, 2) + vy);
     double roc = 0.25 * (u.f[0][a - 1] + u.f[0][a] + u.f[0][c - 1] + u.f[0][c]);
-    roc = 1.0 / sqrt(roc);
+    roc = rcp_ieee(sqrt_ieee(roc));
     const double bxc = 0.5 * (u.f[5][a] + u.f[5][c]);
     const double byc = 0.5 * (u.f[6][c - 1] + u.f[6][c]);
     vxc = fabs(vxc) + fabs(bxc * roc);
     vyc = fabs(vyc) + fabs(byc * roc);
     const double eps = 1e-6;
-    ctx = (vxc + 0.5 * eps) / (vxc + vyc + eps);
+    ctx = quot_ieee(vxc + 0.5 * eps, vxc + vyc + eps);
   }
   w.ctx[s] = ctx;
   sg = 1.0;

@@ -36,7 +36,8 @@ __device__ __forceinline__ void xsweep2d_inl_body(const U2 &u, const W2 &w, cons
   const int j = (int)(q / rl);
   const long s = (long)j * nx + c;
   Stencil S;
-  double m2[3], cxs = 0.0;
+  double cxs = 0.0;
+  bool sup = false;
 #pragma unroll
   for (int m = 0; m < 5; m++) {
     Prim2 P = prim2d_point<ODR>(u, g, bc, c - 2 + m, j);
@@ -48,10 +49,9 @@ __device__ __forceinline__ void xsweep2d_inl_body(const U2 &u, const W2 &w, cons
     S.q[4][m] = P.cy;
     S.q[5][m] = P.bz;
     S.q[6][m] = P.pr;
-    if (m >= 1 && m <= 3) m2[m - 1] = prim2d_m2(g, P);
+    if (m >= 1 && m <= 3) sup |= prim2d_sup(g, P);
     if (m == 2) cxs = P.cx;
   }
-  const bool sup = dmax(m2[0], dmax(m2[1], m2[2])) >= 1.0;
   double vl[7], vr[7];
   recon_p<ODR, MIX>(S, sup, cxs, g.gamma, vl, vr);
   double p[5];
@@ -124,7 +124,7 @@ __device__ __forceinline__ void ysweep2d_inl_body(const U2 &u, const W2 &w, cons
     W[4][m] = P.bz;
     W[5][m] = P.cx;
     W[6][m] = P.pr;
-    supb = (supb & ~(1u << m)) | ((prim2d_m2(g, P) >= 1.0 ? 1u : 0u) << m);
+    supb = (supb & ~(1u << m)) | ((prim2d_sup(g, P) ? 1u : 0u) << m);
   };
   // shock sensor dvx of window row m (row R): aux2d_body's expression
   auto dvx = [&](int R, int m) {
@@ -197,13 +197,13 @@ __device__ __forceinline__ void ysweep2d_inl_body(const U2 &u, const W2 &w, cons
         double vxc = 0.25 * (lvx1 + W[3][1] + lvx2 + W[3][2]);
         double vyc = 0.25 * (lvy1 + W[1][1] + lvy2 + W[1][2]);
         double roc = 0.25 * (lro1 + W[0][1] + lro2 + W[0][2]);
-        roc = 1.0 / sqrt(roc);
+        roc = rcp_ieee(sqrt_ieee(roc));
         const double bxc = 0.5 * (u.f[5][q - N] + u.f[5][q]);
         const double byc = 0.5 * (u.f[6][q - 1] + u.f[6][q]);
         vxc = fabs(vxc) + fabs(bxc * roc);
         vyc = fabs(vyc) + fabs(byc * roc);
         const double eps = 1e-6;
-        w.ctx[q] = (vxc + 0.5 * eps) / (vxc + vyc + eps);
+        w.ctx[q] = quot_ieee(vxc + 0.5 * eps, vxc + vyc + eps);
       }
     }
     double vl[7], ql;

@@ -47,7 +47,7 @@ __device__ __forceinline__ void prim3d_body(U3 u, double *vx_, double *vy_, doub
     c[a] = sg * bc_centre<ODR>(b[-st], b[0], b[st], b[2 * st]);
   }
   const double ro = u.f[0][s];
-  const double iro = 1.0 / ro;
+  const double iro = rcp_ieee(ro);
   const double vx = u.f[1][s] * iro, vy = u.f[2][s] * iro, vz = u.f[3][s] * iro;
   const double v2 = (vx * vx + vy * vy + vz * vz);
   const double b2 = (c[0] * c[0] + c[1] * c[1] + c[2] * c[2]);
@@ -70,13 +70,13 @@ __device__ __forceinline__ double ct_weight(const double *va, const double *vb, 
   double vac = 0.25 * (va[s - sb - sa] + va[s - sb] + va[s - sa] + va[s]);
   double vbc = 0.25 * (vb[s - sb - sa] + vb[s - sb] + vb[s - sa] + vb[s]);
   double roc = 0.25 * (ro[s - sb - sa] + ro[s - sb] + ro[s - sa] + ro[s]);
-  roc = 1.0 / sqrt(roc);
+  roc = rcp_ieee(sqrt_ieee(roc));
   const double bac = 0.5 * (ba[s - sb] + ba[s]);
   const double bbc = 0.5 * (bb[s - sa] + bb[s]);
   vac = fabs(vac) + fabs(bac * roc);
   vbc = fabs(vbc) + fabs(bbc * roc);
   const double eps = 1e-6;
-  return (vac + 0.5 * eps) / (vac + vbc + eps);
+  return quot_ieee(vac + 0.5 * eps, vac + vbc + eps);
 }
 
 // Cell (i, j, k), any cell of the grid.
@@ -98,13 +98,13 @@ __device__ __forceinline__ void aux3d_body(U3 u, const double *vx, const double 
       double vzc = 0.25 * (vz[s - nxy - 1] + vz[s - nxy] + vz[s - 1] + vz[s]);
       double vxc = 0.25 * (vx[s - nxy - 1] + vx[s - nxy] + vx[s - 1] + vx[s]);
       double roc = 0.25 * (u.f[0][s - nxy - 1] + u.f[0][s - nxy] + u.f[0][s - 1] + u.f[0][s]);
-      roc = 1.0 / sqrt(roc);
+      roc = rcp_ieee(sqrt_ieee(roc));
       const double bzc = 0.5 * (u.f[7][s - 1] + u.f[7][s]);
       const double bxc = 0.5 * (u.f[5][s - nxy] + u.f[5][s]);
       vzc = fabs(vzc) + fabs(bzc * roc);
       vxc = fabs(vxc) + fabs(bxc * roc);
       const double eps = 1e-6;
-      w2 = (vzc + 0.5 * eps) / (vzc + vxc + eps);
+      w2 = quot_ieee(vzc + 0.5 * eps, vzc + vxc + eps);
     }
   }
   ct0[s] = w0;
@@ -135,11 +135,11 @@ __device__ __forceinline__ double ct_w4(double a0, double a1, double a2, double 
   double vac = 0.25 * (a0 + a1 + a2 + a3);
   double vbc = 0.25 * (b0 + b1 + b2 + b3);
   double roc = 0.25 * (r0 + r1 + r2 + r3);
-  roc = 1.0 / sqrt(roc);
+  roc = rcp_ieee(sqrt_ieee(roc));
   vac = fabs(vac) + fabs(bac * roc);
   vbc = fabs(vbc) + fabs(bbc * roc);
   const double eps = 1e-6;
-  return (vac + 0.5 * eps) / (vac + vbc + eps);
+  return quot_ieee(vac + 0.5 * eps, vac + vbc + eps);
 }
 
 // aux3d_body on cells (i, j, kc*cz ..): one thread walks cz cells along z and

@@ -507,7 +507,15 @@ MLAU_MIX void riemann(const double (&L)[7], const double (&R)[7], double bn, dou
 // tolerance, not to the reference's bits).
 #pragma clang fp contract(fast)
 namespace fc {
+#define MLAU_RCP(x) (1.0 / (x))
+#define MLAU_QUOT(n, d) ((n) / (d))
+#define MLAU_SQRT(x) sqrt(x)
+#define MLAU_SUB4(x, a, b) (x - 4.0 * a * b)
 #include "mlau_riemann.inc"
+#undef MLAU_RCP
+#undef MLAU_QUOT
+#undef MLAU_SQRT
+#undef MLAU_SUB4
 }  // namespace fc
 #pragma clang fp contract(off)
 

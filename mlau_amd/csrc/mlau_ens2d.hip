@@ -317,7 +317,7 @@ __global__ __launch_bounds__(kFThreads) void k_ens_stage2d(const EnsRec2D *__res
         const double cx = bc_centre<ODR>(0.0, in.f[5][s], in.f[5][s + 1], 0.0);
         const double cy = bc_centre<ODR>(0.0, in.f[6][s], in.f[6][s + nx], 0.0);
         const double ro = in.f[0][s];
-        const double iro = 1.0 / ro;
+        const double iro = rcp_ieee(ro);
         const double vx = in.f[1][s] * iro;
         const double vy = in.f[2][s] * iro;
         const double vz = in.f[3][s] * iro;
@@ -332,7 +332,7 @@ __global__ __launch_bounds__(kFThreads) void k_ens_stage2d(const EnsRec2D *__res
         L.p[FP_VZ][q] = vz;
         L.p[FP_BZ][q] = bz;
         L.p[FP_PR][q] = pr;
-        L.sup[q] = v2 / (gamma * pr * iro) >= 1.0;
+        L.sup[q] = ratio_ge1(v2, gamma * pr * iro);
         L.p[FP_CX][q] = cx;
         L.p[FP_CY][q] = cy;
       }
@@ -493,14 +493,14 @@ __global__ __launch_bounds__(kFThreads) void k_ens_stage2d(const EnsRec2D *__res
         double vxc = 0.25 * (vx[qa - 1] + vx[qa] + vx[q - 1] + vx[q]);
         double vyc = 0.25 * (vy[qa - 1] + vy[qa] + vy[q - 1] + vy[q]);
         double roc = 0.25 * (ro[qa - 1] + ro[qa] + ro[q - 1] + ro[q]);
-        roc = 1.0 / sqrt(roc);
+        roc = rcp_ieee(sqrt_ieee(roc));
         const long s = (long)(c + ej) * nx + (a + ei);
         const double bxc = 0.5 * (in.f[5][s - nx] + in.f[5][s]);
         const double byc = 0.5 * (in.f[6][s - 1] + in.f[6][s]);
         vxc = fabs(vxc) + fabs(bxc * roc);
         vyc = fabs(vyc) + fabs(byc * roc);
         const double eps = 1e-6;
-        ctx = (vxc + 0.5 * eps) / (vxc + vyc + eps);
+        ctx = quot_ieee(vxc + 0.5 * eps, vxc + vyc + eps);
       }
       const double *u4 = &L.x2[0][ej * kFXS + ei], *uc = &L.x2[1][ej * kFXS + ei];
       double a0 = lcal_l<ODR>(0.0, u4[0], u4[kFXS], u4[2 * kFXS], 0.0);
