@@ -31,7 +31,7 @@ struct EnsState {
   long long nstep, max_steps;
   double dtc;                    // CFL step of the current (or, when fixed, the first) step
   int last, fixed;               // fixed: dt from the initial state only (the 1D driver's rule)
-  int halt;                      // set with MLAU_MEMBER_FAILED: the step's updates leave the state alone
+  int halt;                      // no longer running: a step's updates leave the state alone
 };
 
 // Kernel argument of the planning kernels (plain device pointers).
@@ -55,7 +55,8 @@ struct EnsDim {
   long long (*tiles)(const mlau_member &m, int kind, int tune, int variant);  // tiles of a member per kind
   size_t (*member_arrays)(const mlau_grid &g);                   // double arrays per member
   void (*make_record)(void *rec, const mlau_member &m, double *base, size_t per);
-  int (*launch_step)(Ensemble *e, EnsGroup *g);                  // one full step of the group
+  // one full step of the group, the first or the last of those launched together
+  int (*launch_step)(Ensemble *e, EnsGroup *g, bool first, bool last);
   void (*state_ptrs)(const void *rec, double **u0, int *nf, size_t *cells);  // resident state
   int (*variant)(const mlau_member &m, int flags);               // kernel variant (part of the group key)
 };
@@ -150,6 +151,45 @@ void ens_timing_end(Ensemble *e, int k, hipEvent_t a);
     hipLaunchKernelGGL(kernel, grid, block, 0, (e)->cur, __VA_ARGS__);                \
     if ((e)->timing.enabled) ens_timing_end((e), (kid), _ev);                         \
   } while (0)
+
+// dt of a running member from its CFL speed, clipped at its end time.
+__device__ __forceinline__ void ens_dt_slot(const EnsPlan &p, int s)
+{
+  EnsState &S = p.st[s];
+  if (!(S.fixed && S.nstep > 0)) {
+    const double vmax = __longlong_as_double((long long)S.vmax_bits);
+    if (!isfinite(vmax)) {
+      p.stat[s] = MLAU_MEMBER_FAILED;
+      S.halt = 1;
+      S.dt = S.dtdx = S.dtdy = S.dtdz = 0.0;
+      return;
+    }
+    S.dtc = S.cfl * S.dr / vmax;
+  }
+  double dt = S.dtc;
+  if (S.tim + dt >= S.tend) {
+    dt = S.tend - S.tim;
+    S.last = 1;
+  }
+  S.dt = dt;
+  S.dtdx = dt / S.dx;
+  S.dtdy = dt / S.dy;
+  S.dtdz = dt / S.dz;
+}
+
+// End of a running member's step; true while it runs on.
+__device__ __forceinline__ bool ens_advance_slot(const EnsPlan &p, int s)
+{
+  if (p.stat[s] != MLAU_MEMBER_RUNNING) return false;
+  EnsState &S = p.st[s];
+  S.tim = S.last ? S.tend : S.tim + S.dt;
+  S.nstep += 1;
+  if (S.last) p.stat[s] = MLAU_MEMBER_DONE;
+  else if (S.max_steps > 0 && S.nstep >= S.max_steps) p.stat[s] = MLAU_MEMBER_CAPPED;
+  S.vmax_bits = (unsigned long long)__double_as_longlong(S.vfloor);
+  S.halt = p.stat[s] != MLAU_MEMBER_RUNNING;
+  return !S.halt;
+}
 
 // Shared kernels (mlau_ens.hip).
 __global__ void k_ens_plan(EnsPlan p, int ntypes);

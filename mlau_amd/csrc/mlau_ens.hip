@@ -111,43 +111,16 @@ __global__ __launch_bounds__(256) void k_ens_fill(EnsPlan p, int ntypes)
   }
 }
 
-// dt per running member from its CFL speed, clipped at its end time.
 __global__ __launch_bounds__(256) void k_ens_dt(EnsPlan p)
 {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= kEnsSlots || !p.act[s]) return;
-  EnsState &S = p.st[s];
-  if (!(S.fixed && S.nstep > 0)) {
-    const double vmax = __longlong_as_double((long long)S.vmax_bits);
-    if (!isfinite(vmax)) {
-      p.stat[s] = MLAU_MEMBER_FAILED;
-      S.halt = 1;
-      S.dt = S.dtdx = S.dtdy = S.dtdz = 0.0;
-      return;
-    }
-    S.dtc = S.cfl * S.dr / vmax;
-  }
-  double dt = S.dtc;
-  if (S.tim + dt >= S.tend) {
-    dt = S.tend - S.tim;
-    S.last = 1;
-  }
-  S.dt = dt;
-  S.dtdx = dt / S.dx;
-  S.dtdy = dt / S.dy;
-  S.dtdz = dt / S.dz;
+  if (s < kEnsSlots && p.act[s]) ens_dt_slot(p, s);
 }
 
 __global__ __launch_bounds__(256) void k_ens_advance(EnsPlan p)
 {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= kEnsSlots || !p.act[s] || p.stat[s] != MLAU_MEMBER_RUNNING) return;
-  EnsState &S = p.st[s];
-  S.tim = S.last ? S.tend : S.tim + S.dt;
-  S.nstep += 1;
-  if (S.last) p.stat[s] = MLAU_MEMBER_DONE;
-  else if (S.max_steps > 0 && S.nstep >= S.max_steps) p.stat[s] = MLAU_MEMBER_CAPPED;
-  S.vmax_bits = (unsigned long long)__double_as_longlong(S.vfloor);
+  if (s < kEnsSlots && p.act[s]) ens_advance_slot(p, s);
 }
 
 // ------------------------------------------------------------------ timing
@@ -444,7 +417,7 @@ static int launch_steps(Ensemble *e, EnsGroup *G, int n)
 {
   e->cur = G->stream;
   for (int s = 0; s < n; s++) {
-    const int rc = G->D->launch_step(e, G);
+    const int rc = G->D->launch_step(e, G, s == 0, s == n - 1);
     if (rc) return rc;
   }
   return 0;

@@ -1,7 +1,9 @@
 // mlau_ens1d.hip -- batched 1D members of the ensemble engine.
 //
-// Same step structure as the 2D group (plan, fill, CFL, dt, R_K stages,
-// advance); a 1D stage is a sweep (primitives formed per stencil point) and an
+// A 1D member keeps the dt of its first step, so the steps of one launch share
+// one plan, fill, CFL and dt; a member that ends among them is halted, and the
+// bookkeeping between two steps runs in a block of its own of the next first
+// sweep (five launches of little work per step took 60 of its 100 us).  A 1D stage is a sweep (primitives formed per stencil point) and an
 // update that also runs the open boundary on stage 0 and writes periodic
 // ghosts with their source cells, as the single-grid path; at odr <= 2 with
 // rk >= 2 the later stages are one launch each (k_ens_stage1d, flux and update
@@ -101,11 +103,16 @@ __global__ __launch_bounds__(256) void k_ens_cfl1d(const EnsRec1D *__restrict__ 
 template <int ODR, int FLUX, int MIX>
 __global__ __launch_bounds__(256) void k_ens_sweep1d(const EnsRec1D *__restrict__ rec,
                                                      const int2 *__restrict__ tiles, const int *__restrict__ count,
-                                                     int sin)
+                                                     int sin, EnsPlan p, int next)
 {
   ENS_LOOP(T1_SWEEP)
     sweep1d_body<ODR, FLUX, MIX>(sin ? R.u1 : R.u0, R.w, R.g, l_, threadIdx.x);
   }
+  // The first sweep of a step reads no dt: its last block, which has no tiles,
+  // ends the members' previous step and forms this one's dt meanwhile.
+  if (next && blockIdx.x == gridDim.x - 1)
+    for (int s = threadIdx.x; s < kEnsSlots; s += blockDim.x)
+      if (p.act[s] && ens_advance_slot(p, s)) ens_dt_slot(p, s);
 }
 
 // stage 0 only: the stage input is u0; ghosts go to u0 and u1
@@ -113,7 +120,7 @@ __global__ __launch_bounds__(64) void k_ens_openbc1d(const EnsRec1D *__restrict_
                                                      const int2 *__restrict__ tiles, const int *__restrict__ count)
 {
   ENS_LOOP(T1_OBC)
-    if (st[e_.x].halt) continue;  // member failed at this step's CFL check
+    if (st[e_.x].halt) continue;  // failed at this step's CFL check, or ended
     (void)l_;
     openbc1d_body(R.u0, R.u0, R.u1, R.g, st[e_.x].dtdx, threadIdx.x);
   }
@@ -129,7 +136,7 @@ __global__ __launch_bounds__(256) void k_ens_update1d(const EnsRec1D *__restrict
                                                       double rb, int obc)
 {
   ENS_LOOP(T1_UPD)
-    if (st[e_.x].halt) continue;  // member failed at this step's CFL check
+    if (st[e_.x].halt) continue;  // failed at this step's CFL check, or ended
     const U1d in = sin ? R.u1 : R.u0, out = sout ? R.u1 : R.u0;
     if (R.bc1d == MLAU_BC1D_PERIODIC)
       update1d_body<ODR, true>(in, R.u0, out, R.w, R.g, st[e_.x].dtdx, ra, rb, l_, threadIdx.x);
@@ -139,7 +146,7 @@ __global__ __launch_bounds__(256) void k_ens_update1d(const EnsRec1D *__restrict
   if (!obc) return;
   tiles = otiles;
   ENS_LOOP(T1_OBC)
-    if (st[e_.x].halt) continue;  // member failed at this step's CFL check
+    if (st[e_.x].halt) continue;  // failed at this step's CFL check, or ended
     (void)l_;
     openbc1d_body(R.u0, R.u0, R.u1, R.g, st[e_.x].dtdx, threadIdx.x);
   }
@@ -154,7 +161,7 @@ __global__ __launch_bounds__(256) void k_ens_stage1d(const EnsRec1D *__restrict_
                                                      int sin, int sout, double ra, double rb)
 {
   ENS_LOOP(T1_FUSE)
-    if (st[e_.x].halt) continue;  // member failed at this step's CFL check
+    if (st[e_.x].halt) continue;  // failed at this step's CFL check, or ended
     const U1d in = ubuf1(R, sin), out = ubuf1(R, sout);
     const double dtdx = st[e_.x].dtdx;
     const unsigned wave = l_ * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -174,16 +181,21 @@ static unsigned pers_blocks1(const Ensemble *e)
 }
 
 template <int ODR, int MIX>
-static void sweep1d(Ensemble *e, int flux, unsigned pb, const EnsRec1D *rec, const EnsPlan &p, int sin)
+static void sweep1d(Ensemble *e, int flux, unsigned pb, const EnsRec1D *rec, const EnsPlan &p, int sin, int next)
 {
+  pb += next;  // one block more than the whole sets of kXcds that share the tiles (pers_range)
   const int2 *t = (const int2 *)p.tiles[T1_SWEEP];
   const int *cnt = p.count;
   const dim3 b(256);
   switch (flux) {
-  case FLUX_MLAU: ENS_LAUNCH(e, E_XSWEEP, (k_ens_sweep1d<ODR, FLUX_MLAU, MIX>), dim3(pb), b, rec, t, cnt, sin); break;
-  case FLUX_ROE: ENS_LAUNCH(e, E_XSWEEP, (k_ens_sweep1d<ODR, FLUX_ROE, MIX>), dim3(pb), b, rec, t, cnt, sin); break;
-  case FLUX_HLLD: ENS_LAUNCH(e, E_XSWEEP, (k_ens_sweep1d<ODR, FLUX_HLLD, MIX>), dim3(pb), b, rec, t, cnt, sin); break;
-  default: ENS_LAUNCH(e, E_XSWEEP, (k_ens_sweep1d<ODR, FLUX_LHLLD, MIX>), dim3(pb), b, rec, t, cnt, sin); break;
+  case FLUX_MLAU: ENS_LAUNCH(e, E_XSWEEP, (k_ens_sweep1d<ODR, FLUX_MLAU, MIX>), dim3(pb), b, rec, t, cnt, sin, p, next);
+    break;
+  case FLUX_ROE: ENS_LAUNCH(e, E_XSWEEP, (k_ens_sweep1d<ODR, FLUX_ROE, MIX>), dim3(pb), b, rec, t, cnt, sin, p, next);
+    break;
+  case FLUX_HLLD: ENS_LAUNCH(e, E_XSWEEP, (k_ens_sweep1d<ODR, FLUX_HLLD, MIX>), dim3(pb), b, rec, t, cnt, sin, p, next);
+    break;
+  default: ENS_LAUNCH(e, E_XSWEEP, (k_ens_sweep1d<ODR, FLUX_LHLLD, MIX>), dim3(pb), b, rec, t, cnt, sin, p, next);
+    break;
   }
 }
 
@@ -213,17 +225,19 @@ static void stage1d(Ensemble *e, int flux, unsigned pb, const EnsRec1D *rec, con
 }
 
 template <int ODR, int MIX>
-static int step1d_group(Ensemble *e, EnsGroup *G)
+static int step1d_group(Ensemble *e, EnsGroup *G, bool first, bool last)
 {
   const EnsPlan &p = G->p;
   const EnsRec1D *rec = (const EnsRec1D *)G->rec;
   const unsigned pb = pers_blocks1(e);
   const dim3 b256(256), b64(64), slots(kEnsSlots / 256);
   const int *cnt = p.count;
-  ENS_LAUNCH(e, E_PLAN, k_ens_plan, dim3(1), dim3(kPlanThreads), p, (int)T1_N);
-  ENS_LAUNCH(e, E_FILL, k_ens_fill, dim3(kEnsSlots), b256, p, (int)T1_N);
-  ENS_LAUNCH(e, E_CFL, k_ens_cfl1d, dim3(pb), b256, rec, p.st, (const int2 *)p.tiles[T1_CFL], cnt);
-  ENS_LAUNCH(e, E_DT, k_ens_dt, slots, b256, p);
+  if (first) {
+    ENS_LAUNCH(e, E_PLAN, k_ens_plan, dim3(1), dim3(kPlanThreads), p, (int)T1_N);
+    ENS_LAUNCH(e, E_FILL, k_ens_fill, dim3(kEnsSlots), b256, p, (int)T1_N);
+    ENS_LAUNCH(e, E_CFL, k_ens_cfl1d, dim3(pb), b256, rec, p.st, (const int2 *)p.tiles[T1_CFL], cnt);
+    ENS_LAUNCH(e, E_DT, k_ens_dt, slots, b256, p);
+  }
   const int R_K = G->rk;
   const double rkf[3][2] = {{0.0, 1.0}, {0.5 + (R_K - 2) * 0.25, 0.5 - (R_K - 2) * 0.25}, {1. / 3., 2. / 3.}};
   for (int rk = 0; rk < R_K; rk++) {
@@ -235,7 +249,7 @@ static int step1d_group(Ensemble *e, EnsGroup *G)
     }
     const int sin = (rk == 0) ? 0 : 1;
     const int sout = (rk == R_K - 1) ? 0 : 1;
-    sweep1d<ODR, MIX>(e, G->flux, pb, rec, p, sin);
+    sweep1d<ODR, MIX>(e, G->flux, pb, rec, p, sin, rk == 0 && !first);
     const int obc = rk == 0 && R_K > 1;  // RK1 updates in place: boundary first, separately
     if (rk == 0 && !obc)
       ENS_LAUNCH(e, E_BC, k_ens_openbc1d, dim3(e->cus), b64, rec, (const EnsState *)p.st,
@@ -244,11 +258,11 @@ static int step1d_group(Ensemble *e, EnsGroup *G)
                (const int2 *)p.tiles[T1_UPD], (const int2 *)p.tiles[T1_OBC], cnt, sin, sout, rkf[rk][0], rkf[rk][1],
                obc);
   }
-  ENS_LAUNCH(e, E_ADVANCE, k_ens_advance, slots, b256, p);
+  if (last) ENS_LAUNCH(e, E_ADVANCE, k_ens_advance, slots, b256, p);
   return (int)hipGetLastError();
 }
 
-typedef int (*EnsStepFn)(Ensemble *, EnsGroup *);
+typedef int (*EnsStepFn)(Ensemble *, EnsGroup *, bool, bool);
 
 template <int ODR>
 static EnsStepFn pick1_odr(int precision)
@@ -260,7 +274,7 @@ static EnsStepFn pick1_odr(int precision)
   }
 }
 
-static int launch1d(Ensemble *e, EnsGroup *G)
+static int launch1d(Ensemble *e, EnsGroup *G, bool first, bool last)
 {
   EnsStepFn fn;
   switch (G->odr) {
@@ -269,7 +283,7 @@ static int launch1d(Ensemble *e, EnsGroup *G)
   case 3: fn = pick1_odr<3>(G->precision); break;
   default: fn = pick1_odr<4>(G->precision); break;
   }
-  return fn(e, G);
+  return fn(e, G, first, last);
 }
 
 static const EnsDim kDim1d = {sizeof(EnsRec1D), T1_N, tiles1d_member, arrays1d, record1d, launch1d, state1d,

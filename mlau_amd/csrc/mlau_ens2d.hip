@@ -673,7 +673,7 @@ static EnsStepFn pick_odr(int ctw, int precision, int tune)
   }
 }
 
-static int launch2d(Ensemble *e, EnsGroup *G)
+static int launch2d(Ensemble *e, EnsGroup *G, bool, bool)
 {
   EnsStepFn fn;
   switch (G->odr) {

@@ -321,7 +321,7 @@ static EnsStepFn pick3_odr(int ctw, int precision)
   }
 }
 
-static int launch3d(Ensemble *e, EnsGroup *G)
+static int launch3d(Ensemble *e, EnsGroup *G, bool, bool)
 {
   EnsStepFn fn;
   switch (G->odr) {
