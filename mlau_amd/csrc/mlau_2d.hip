@@ -59,11 +59,10 @@ __global__ __launch_bounds__(256) void k_xsweep2d(U2 u, W2 w, G2 g)
   xsweep2d_body<ODR, FLUX, MIX>(u, w, g, W, threadIdx.x & 63);
 }
 
-template <int ODR, int FLUX, int MIX, bool SPLIT>
+template <int ODR, int FLUX, int MIX>
 __global__ __launch_bounds__(64) void k_ysweep2d(U2 u, W2 w, G2 g, int ch)
 {
-  ysweep2d_body<ODR, FLUX, MIX, SPLIT>(u, w, g, ch, march_mid(ch, blockIdx.y, kMarch), blockIdx.x, blockIdx.y,
-                                        threadIdx.x);
+  ysweep2d_body<ODR, FLUX, MIX, false>(u, w, g, ch, false, blockIdx.x, blockIdx.y, threadIdx.x);
 }
 
 template <int ODR>
@@ -102,11 +101,37 @@ __global__ __launch_bounds__(256) void k_xsweep2d_inl(U2 u, W2 w, G2 g)
   xsweep2d_inl_body<ODR, FLUX, MIX>(u, w, g, W, threadIdx.x & 63);
 }
 
-template <int ODR, int FLUX, int MIX, int CTW, bool SPLIT>
+template <int ODR, int FLUX, int MIX, int CTW>
 __global__ __launch_bounds__(64) void k_ysweep2d_inl(U2 u, W2 w, G2 g, int ch)
 {
-  ysweep2d_inl_body<ODR, FLUX, MIX, CTW, SPLIT>(u, w, g, ch, march_mid(ch, blockIdx.y, kMarch), blockIdx.x,
-                                                blockIdx.y, threadIdx.x);
+  ysweep2d_inl_body<ODR, FLUX, MIX, CTW, false>(u, w, g, ch, false, blockIdx.x, blockIdx.y, threadIdx.x);
+}
+
+// Both sweeps in one launch, as all stages run them: blocks below `ny` are
+// y-sweep blocks (px pieces of a row by marches), the others one x-sweep
+// wavefront each.  The sweeps share no output, and both fit two wavefronts to
+// a SIMD.  Against two launches on two streams, where a fork and a join
+// wait on each other's events, 8 steps, us: 64^2 964 -> 599, 256^2 1278 -> 1041,
+// 1024^2 6898 -> 6604, 2048^2 26117 -> 25610; mixed 256^2 1133 -> 826, 1024^2 5587 ->
+// 4797 (the x sweep's third wavefront lost nothing); walls 512^2 1991 -> 1825.
+template <int ODR, int FLUX, int MIX, int CTW, bool SPLIT>
+__global__ __launch_bounds__(64) void k_sweeps2d_inl(U2 u, W2 w, G2 g, int ch, unsigned px, unsigned ny)
+{
+  const unsigned b = blockIdx.x;
+  if (b < ny)
+    ysweep2d_inl_body<ODR, FLUX, MIX, CTW, SPLIT>(u, w, g, ch, march_mid(ch, b / px, kMarch), b % px, b / px,
+                                                  threadIdx.x);
+  else
+    xsweep2d_inl_body<ODR, FLUX, MIX>(u, w, g, (long)(b - ny), threadIdx.x);
+}
+template <int ODR, int FLUX, int MIX, bool SPLIT>
+__global__ __launch_bounds__(64) void k_sweeps2d(U2 u, W2 w, G2 g, int ch, unsigned px, unsigned ny)
+{
+  const unsigned b = blockIdx.x;
+  if (b < ny)
+    ysweep2d_body<ODR, FLUX, MIX, SPLIT>(u, w, g, ch, march_mid(ch, b / px, kMarch), b % px, b / px, threadIdx.x);
+  else
+    xsweep2d_body<ODR, FLUX, MIX>(u, w, g, (long)(b - ny), threadIdx.x);
 }
 
 // CT weight 1/2 at corners 3..nx-3 x 3..ny-3 (no upwind weighting)
@@ -174,22 +199,28 @@ static int ychunk(const Handle *h, const G2 &g)
                               h->s.precision != MLAU_FP64);
 }
 
+// Per-kernel timing and tune bit 6 launch the sweeps one by one.
+static bool one_by_one(const Handle *h) { return h->timing.enabled || (h->tune & 64); }
+
 template <int ODR, int FLUX, int MIX>
 static void sweeps2d(Handle *h, const U2 &in, const W2 &w, const G2 &g)
 {
-  const dim3 gx((unsigned)((xsweep_waves(g.ny, g.nx) + 3) / 4));
-  Side sd(h);  // the y sweep beside the x sweep
-  sd.fork(1);
-  MLAU_LAUNCH(h, K_XSWEEP2D, (k_xsweep2d<ODR, FLUX, MIX>), gx, dim3(256), in, w, g);
-  sd.enter(0);
-  const int ch = whole_march<FLUX, MIX> ? kMarch : ychunk(h, g);
-  const dim3 gy((g.nx + 63) / 64, (g.ny - 5 + ch - 1) / ch);
+  const unsigned px = (g.nx + 63) / 64;
+  const long xw = xsweep_waves(g.ny, g.nx);
+  int ch = whole_march<FLUX, MIX> ? kMarch : ychunk(h, g);
+  if (one_by_one(h)) {
+    if (split_march<MIX>(ch)) ch = kMarch;
+    MLAU_LAUNCH(h, K_XSWEEP2D, (k_xsweep2d<ODR, FLUX, MIX>), dim3((unsigned)((xw + 3) / 4)), dim3(256), in, w, g);
+    MLAU_LAUNCH(h, K_YSWEEP2D, (k_ysweep2d<ODR, FLUX, MIX>), dim3(px, (g.ny - 5 + ch - 1) / ch), dim3(64), in, w, g,
+                ch);
+    return;
+  }
+  const unsigned nyb = px * ((g.ny - 5 + ch - 1) / ch);
+  const dim3 gr(nyb + (unsigned)xw);
   if (split_march<MIX>(ch))
-    MLAU_LAUNCH(h, K_YSWEEP2D, (k_ysweep2d<ODR, FLUX, MIX, MIX != MLAU_FP64>), gy, dim3(64), in, w, g, ch);
+    MLAU_LAUNCH(h, K_SWEEPS2D, (k_sweeps2d<ODR, FLUX, MIX, MIX != MLAU_FP64>), gr, dim3(64), in, w, g, ch, px, nyb);
   else
-    MLAU_LAUNCH(h, K_YSWEEP2D, (k_ysweep2d<ODR, FLUX, MIX, false>), gy, dim3(64), in, w, g, ch);
-  sd.leave();
-  sd.join();
+    MLAU_LAUNCH(h, K_SWEEPS2D, (k_sweeps2d<ODR, FLUX, MIX, false>), gr, dim3(64), in, w, g, ch, px, nyb);
 }
 
 template <int ODR, int FLUX, int MIX>
@@ -226,12 +257,25 @@ static void stage2d(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const 
 }
 
 template <int ODR, int FLUX, int MIX, int CTW>
-static void launch_ysweep_inl(Handle *h, const U2 &in, const W2 &w, const G2 &g, dim3 gy, int ch)
+static void sweeps2d_inl(Handle *h, const U2 &in, const W2 &w, const G2 &g)
 {
+  const unsigned px = (g.nx + 63) / 64;
+  const long xw = xsweep_waves(g.ny, g.nx);
+  int ch = ychunk(h, g);
+  if (one_by_one(h)) {
+    if (split_march<MIX>(ch)) ch = kMarch;
+    MLAU_LAUNCH(h, K_XSW2D_INL, (k_xsweep2d_inl<ODR, FLUX, MIX>), dim3((unsigned)((xw + 3) / 4)), dim3(256), in, w, g);
+    MLAU_LAUNCH(h, K_YSW2D_INL, (k_ysweep2d_inl<ODR, FLUX, MIX, CTW>), dim3(px, (g.ny - 5 + ch - 1) / ch), dim3(64),
+                in, w, g, ch);
+    return;
+  }
+  const unsigned nyb = px * ((g.ny - 5 + ch - 1) / ch);
+  const dim3 gr(nyb + (unsigned)xw);
   if (split_march<MIX>(ch))
-    MLAU_LAUNCH(h, K_YSW2D_INL, (k_ysweep2d_inl<ODR, FLUX, MIX, CTW, MIX != MLAU_FP64>), gy, dim3(64), in, w, g, ch);
+    MLAU_LAUNCH(h, K_SWEEPS2D, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, MIX != MLAU_FP64>), gr, dim3(64), in, w, g, ch, px,
+                nyb);
   else
-    MLAU_LAUNCH(h, K_YSW2D_INL, (k_ysweep2d_inl<ODR, FLUX, MIX, CTW, false>), gy, dim3(64), in, w, g, ch);
+    MLAU_LAUNCH(h, K_SWEEPS2D, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, false>), gr, dim3(64), in, w, g, ch, px, nyb);
 }
 
 // Periodic grids (with room for the ghost images written by the update): the
@@ -240,17 +284,8 @@ template <int ODR, int FLUX, int MIX>
 static void stage2d_inl(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const W2 &w, const G2 &g, double ra,
                         double rb, int adv)
 {
-  const dim3 gx((unsigned)((xsweep_waves(g.ny, g.nx) + 3) / 4));
-  Side sd(h);  // the y sweep beside the x sweep
-  sd.fork(1);
-  MLAU_LAUNCH(h, K_XSW2D_INL, (k_xsweep2d_inl<ODR, FLUX, MIX>), gx, dim3(256), in, w, g);
-  sd.enter(0);
-  const int ch = ychunk(h, g);
-  const dim3 gy((g.nx + 63) / 64, (g.ny - 5 + ch - 1) / ch);
-  if (h->s.ctw) launch_ysweep_inl<ODR, FLUX, MIX, 1>(h, in, w, g, gy, ch);
-  else launch_ysweep_inl<ODR, FLUX, MIX, 0>(h, in, w, g, gy, ch);
-  sd.leave();
-  sd.join();
+  if (h->s.ctw) sweeps2d_inl<ODR, FLUX, MIX, 1>(h, in, w, g);
+  else sweeps2d_inl<ODR, FLUX, MIX, 0>(h, in, w, g);
   if (!h->s.ctw) {  // constant weight 1/2 (aux2d_body with CTW 0) over the corners the E-field reads
     const dim3 gc(region_pieces(g.nx - 5, g.ny - 5));
     MLAU_LAUNCH(h, K_AUX2D, k_ctx_half2d, gc, dim3(256), w, g);

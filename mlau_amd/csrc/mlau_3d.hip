@@ -71,9 +71,36 @@ __global__ __launch_bounds__(256) void k_xsweep3d(Sw3 w, G3 g)
   xsweep3d_body<ODR, FLUX, MIX>(w, g, W, threadIdx.x & 63);
 }
 
+// All three sweeps in one launch, as all stages run them: blocks below yb march
+// along y, those below yb + zb along z, the others are one x-sweep wavefront
+// each.  Against three launches on three streams with their fork and join, 8 steps, us:
+// 24^3 1654 -> 1081, 48^3 2823 -> 2352, 96^3 11773 -> 11463, 128^3 26804 -> 26623;
+// mixed 32^3 1766 -> 1180, 128^3 21044 -> 20492.
+template <int ODR, int FLUX, int MIX, bool SPLIT>
+__global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_sweeps3d(Sw3 wx, Sw3 wy, Sw3 wz, G3 g, int chy, int chz,
+                                                                unsigned yb, unsigned zb)
+{
+  const unsigned b = blockIdx.x;
+  if (b < yb) {
+    const unsigned pieces = (unsigned)(((long)g.nx * g.nz + 63) / 64), c = b / pieces;
+    const long p = (long)(b % pieces) * 64 + threadIdx.x;
+    if (p < (long)g.nx * g.nz)
+      msweep3d_body<ODR, FLUX, 1, MIX, SPLIT>(wy, g, chy, march_mid(chy, c, kMarch), (int)(p % g.nx), c,
+                                              (int)(p / g.nx));
+  } else if (b < yb + zb) {
+    const unsigned pieces = (unsigned)(((long)g.nx * g.ny + 63) / 64), c = (b - yb) / pieces;
+    const long p = (long)((b - yb) % pieces) * 64 + threadIdx.x;
+    if (p < (long)g.nx * g.ny)
+      msweep3d_body<ODR, FLUX, 2, MIX, SPLIT>(wz, g, chz, march_mid(chz, c, kMarch), (int)(p % g.nx), c,
+                                              (int)(p / g.nx));
+  } else {
+    xsweep3d_body<ODR, FLUX, MIX>(wx, g, (long)(b - yb - zb), threadIdx.x);
+  }
+}
+
 // y/z sweeps: lanes over the flattened (i, third coordinate) columns; blocks
 // are (column piece, chunk along the sweep axis)
-template <int ODR, int FLUX, int AX, int MIX, bool SPLIT>
+template <int ODR, int FLUX, int AX, int MIX>
 __global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_msweep3d(Sw3 w, G3 g, int ch)
 {
   const long nc = (AX == 1) ? g.nz : g.ny;
@@ -81,7 +108,7 @@ __global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_msweep3d(Sw3 w, G3 g, int
   const long p = (long)(blockIdx.x % pieces) * 64 + threadIdx.x;
   if (p >= g.nx * nc) return;
   const unsigned c = blockIdx.x / pieces;
-  msweep3d_body<ODR, FLUX, AX, MIX, SPLIT>(w, g, ch, march_mid(ch, c, kMarch), (int)(p % g.nx), c, (int)(p / g.nx));
+  msweep3d_body<ODR, FLUX, AX, MIX, false>(w, g, ch, false, (int)(p % g.nx), c, (int)(p / g.nx));
 }
 
 template <int ODR>
@@ -192,19 +219,6 @@ static Sw3 sweep_view(Handle *h, const U3 &in, int ax)
   return w;
 }
 
-template <int ODR, int FLUX, int AX, int MIX>
-static void launch_march(Handle *h, int kid, const Sw3 &w, const G3 &g, long pieces, int faces, int ch)
-{
-  const dim3 gr((unsigned)(pieces * ((faces + ch - 1) / ch)));
-  if constexpr (MIX != MLAU_FP64) {
-    if (ch < kMarch) {
-      MLAU_LAUNCH(h, kid, (k_msweep3d<ODR, FLUX, AX, MIX, true>), gr, dim3(64), w, g, ch);
-      return;
-    }
-  }
-  MLAU_LAUNCH(h, kid, (k_msweep3d<ODR, FLUX, AX, MIX, false>), gr, dim3(64), w, g, ch);
-}
-
 template <int ODR, int FLUX, int MIX>
 static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double ra, double rb, int adv)
 {
@@ -235,16 +249,23 @@ static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double
   const bool whole = whole_march<FLUX, MIX>;
   const int chy = whole ? kMarch : march_chunk(yw, ny - 5, xw + zw * nz, 0.2, kMarch, MIX != MLAU_FP64);
   const int chz = whole ? kMarch : march_chunk(zw, nz - 5, xw + yw * ny, 0.2, kMarch, MIX != MLAU_FP64);
-  Side sd(h);  // the y and z sweeps beside the x sweep
-  sd.fork(2);
-  MLAU_LAUNCH(h, K_XSWEEP3D, (k_xsweep3d<ODR, FLUX, MIX>), dim3((unsigned)((xw + 3) / 4)), b256,
-              sweep_view(h, in, 0), g);
-  sd.enter(0);
-  launch_march<ODR, FLUX, 1, MIX>(h, K_YSWEEP3D, sweep_view(h, in, 1), g, yw, ny - 5, chy);
-  sd.enter(1);
-  launch_march<ODR, FLUX, 2, MIX>(h, K_ZSWEEP3D, sweep_view(h, in, 2), g, zw, nz - 5, chz);
-  sd.leave();
-  sd.join();
+  const Sw3 wx = sweep_view(h, in, 0), wy = sweep_view(h, in, 1), wz = sweep_view(h, in, 2);
+  if (h->timing.enabled || (h->tune & 64)) {  // per-kernel timing and tune bit 6: one by one
+    const int cy = MIX != MLAU_FP64 ? kMarch : chy, cz_ = MIX != MLAU_FP64 ? kMarch : chz;
+    MLAU_LAUNCH(h, K_XSWEEP3D, (k_xsweep3d<ODR, FLUX, MIX>), dim3((unsigned)((xw + 3) / 4)), b256, wx, g);
+    MLAU_LAUNCH(h, K_YSWEEP3D, (k_msweep3d<ODR, FLUX, 1, MIX>), dim3((unsigned)(yw * ((ny - 5 + cy - 1) / cy))),
+                dim3(64), wy, g, cy);
+    MLAU_LAUNCH(h, K_ZSWEEP3D, (k_msweep3d<ODR, FLUX, 2, MIX>), dim3((unsigned)(zw * ((nz - 5 + cz_ - 1) / cz_))),
+                dim3(64), wz, g, cz_);
+  } else {
+    const unsigned yb = (unsigned)(yw * ((ny - 5 + chy - 1) / chy)), zb = (unsigned)(zw * ((nz - 5 + chz - 1) / chz));
+    const dim3 gr(yb + zb + (unsigned)xw);
+    if (MIX != MLAU_FP64 && (chy < kMarch || chz < kMarch))
+      MLAU_LAUNCH(h, K_SWEEPS3D, (k_sweeps3d<ODR, FLUX, MIX, MIX != MLAU_FP64>), gr, dim3(64), wx, wy, wz, g, chy, chz,
+                  yb, zb);
+    else
+      MLAU_LAUNCH(h, K_SWEEPS3D, (k_sweeps3d<ODR, FLUX, MIX, false>), gr, dim3(64), wx, wy, wz, g, chy, chz, yb, zb);
+  }
   Edge3 e;
   e.fxt = h->fx[4]; e.fxu = h->fx[5]; e.fcx0 = h->fcx[0]; e.fcx1 = h->fcx[1];
   e.fyt = h->fy[4]; e.fyu = h->fy[5]; e.fcy0 = h->fcy[0]; e.fcy1 = h->fcy[1];
