@@ -198,18 +198,9 @@ __device__ __forceinline__ void openbc1d_cell(const double (&q)[7][2], const G1d
   vals[6] = bz;
 }
 
-// thread 0 = left edge, thread 1 = right edge.  Reads the stage input and
-// writes the boundary ghosts of every buffer in `dst` (the stage output and
-// the step-start state, so later stages and the final state both see them).
-__device__ __forceinline__ void openbc1d_body(U1d in, U1d dst0, U1d dst1, G1d g, double dtdx, unsigned side)
+// Primitives (ro, vx, vy, vz, by, bz, pr) of cells si and so.
+__device__ __forceinline__ void prim1d_pair(const U1d &in, int si, int so, double gamma, double bx, double (&q)[7][2])
 {
-  if (side > 1) return;
-  const int nx = g.nx, xoff = g.xoff;
-  const int sgn = side == 0 ? 1 : -1;
-  const int si = side == 0 ? xoff : nx - xoff - 1;
-  const int so = si - sgn;
-  const double bx = g.bx, gamma = g.gamma;
-  double q[7][2];
   const int idx[2] = {si, so};
   for (int j = 0; j < 2; j++) {
     const int ss = idx[j];
@@ -227,6 +218,20 @@ __device__ __forceinline__ void openbc1d_body(U1d in, U1d dst0, U1d dst1, G1d g,
     q[5][j] = bz;
     q[6][j] = (gamma - 1.0) * (in.f[4][ss] - 0.5 * (ro * v2 + b2));
   }
+}
+
+// thread 0 = left edge, thread 1 = right edge.  Reads the stage input and
+// writes the boundary ghosts of every buffer in `dst` (the stage output and
+// the step-start state, so later stages and the final state both see them).
+__device__ __forceinline__ void openbc1d_body(U1d in, U1d dst0, U1d dst1, G1d g, double dtdx, unsigned side)
+{
+  if (side > 1) return;
+  const int nx = g.nx, xoff = g.xoff;
+  const int sgn = side == 0 ? 1 : -1;
+  const int si = side == 0 ? xoff : nx - xoff - 1;
+  const int so = si - sgn;
+  double q[7][2];
+  prim1d_pair(in, si, so, g.gamma, g.bx, q);
   double vals[7];
   openbc1d_cell<false>(q, g, dtdx, side, vals);
   U1d *dsts[2] = {&dst0, &dst1};

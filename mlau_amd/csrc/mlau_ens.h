@@ -59,6 +59,10 @@ struct EnsDim {
   int (*launch_step)(Ensemble *e, EnsGroup *g, bool first, bool last);
   void (*state_ptrs)(const void *rec, double **u0, int *nf, size_t *cells);  // resident state
   int (*variant)(const mlau_member &m, int flags);               // kernel variant (part of the group key)
+  // all n steps launched together, for groups whose kernels take several steps (-1: step by step),
+  // and the steps of a group's graph (Ensemble::gsteps without it)
+  int (*launch_many)(Ensemble *e, EnsGroup *g, int n) = nullptr;
+  int (*graph_steps)(const Ensemble *e, const EnsGroup *g) = nullptr;
 };
 const EnsDim *ens_dim1d();
 const EnsDim *ens_dim2d();
@@ -89,8 +93,8 @@ struct EnsGroup {
   // the group's steps run on its own stream, beside the other groups' steps
   hipStream_t stream = nullptr;
   hipEvent_t ev_start = nullptr, ev_done = nullptr;
-  hipGraphExec_t gx = nullptr;              // graph of Ensemble::gsteps steps (captured on first use)
-  int gx_tune = -1;                         // tuning the graph was captured with
+  hipGraphExec_t gx = nullptr;              // graph of gx_steps steps (captured on first use)
+  int gx_tune = -1, gx_steps = 0;           // tuning and steps the graph was captured with
   int launched = 0;                         // steps in the launch in flight
   double step_ms = 0.0;                     // measured time per step (0: not yet measured)
 };

@@ -416,6 +416,10 @@ static long long member_tiles_max(const EnsDim *D, const mlau_member &m, int k, 
 static int launch_steps(Ensemble *e, EnsGroup *G, int n)
 {
   e->cur = G->stream;
+  if (G->D->launch_many) {
+    const int rc = G->D->launch_many(e, G, n);
+    if (rc >= 0) return rc;
+  }
   for (int s = 0; s < n; s++) {
     const int rc = G->D->launch_step(e, G, s == 0, s == n - 1);
     if (rc) return rc;
@@ -431,10 +435,16 @@ static void graph_drop(Ensemble *e)
   }
 }
 
-// The group's graph of gsteps steps for the current tuning (captured on first use).
+static int graph_steps(const Ensemble *e, const EnsGroup *G)
+{
+  return G->D->graph_steps ? G->D->graph_steps(e, G) : e->gsteps;
+}
+
+// The group's graph of graph_steps steps for the current tuning (captured on first use).
 static int graph_get(Ensemble *e, EnsGroup *G, hipGraphExec_t *out)
 {
-  if (G->gx && G->gx_tune == e->tune) {
+  const int gs = graph_steps(e, G);
+  if (G->gx && G->gx_tune == e->tune && G->gx_steps == gs) {
     *out = G->gx;
     return MLAU_OK;
   }
@@ -443,7 +453,7 @@ static int graph_get(Ensemble *e, EnsGroup *G, hipGraphExec_t *out)
   hipGraph_t g = nullptr;
   if (hipStreamBeginCapture(G->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
     return fail(MLAU_ERR_HIP, "hipStreamBeginCapture failed");
-  const int rc = launch_steps(e, G, e->gsteps);
+  const int rc = launch_steps(e, G, gs);
   const hipError_t ec = hipStreamEndCapture(G->stream, &g);
   if (rc || ec != hipSuccess) {
     if (g) hipGraphDestroy(g);
@@ -455,6 +465,7 @@ static int graph_get(Ensemble *e, EnsGroup *G, hipGraphExec_t *out)
   if (ei != hipSuccess) return hip_fail(ei, "hipGraphInstantiate");
   G->gx = x;
   G->gx_tune = e->tune;
+  G->gx_steps = gs;
   *out = x;
   return MLAU_OK;
 }
@@ -820,16 +831,17 @@ int mlau_ens_launch(mlau_ensemble *e, int nsteps)
     G->launched = 0;
     if (G->nrun == 0) continue;
     int left = group_steps(e, G, nsteps);
+    const int gs = graph_steps(e, G);
     hipGraphExec_t x = nullptr;
-    if (graph && (left >= e->gsteps || left == 0) && (rc = graph_get(e, G, &x))) break;  // zero steps: capture only
+    if (graph && (left >= gs || left == 0) && (rc = graph_get(e, G, &x))) break;  // zero steps: capture only
     if (left == 0) continue;
     G->launched = left;
     hipError_t he = hipStreamWaitEvent(G->stream, e->ctl_ev, 0);  // after the control writes
     if (he == hipSuccess && serial && prev) he = hipStreamWaitEvent(G->stream, prev->ev_done, 0);
     if (he == hipSuccess) he = hipEventRecord(G->ev_start, G->stream);
-    while (he == hipSuccess && x && left >= e->gsteps) {
+    while (he == hipSuccess && x && left >= gs) {
       he = hipGraphLaunch(x, G->stream);
-      left -= e->gsteps;
+      left -= gs;
     }
     if (he == hipSuccess && left > 0) he = (hipError_t)launch_steps(e, G, left);
     if (he == hipSuccess) he = hipEventRecord(G->ev_done, G->stream);

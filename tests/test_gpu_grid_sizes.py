@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import mlau_amd as M
+from mlau_amd import ensemble as E
 from mlau_amd import problems as P
 from oracle import oracle as O
 
@@ -100,3 +101,40 @@ def test_1d_cfl_loop(gpu, bc, steps):
     assert s.time()[1] == dt
     assert_same(s.download(), f_o, "1D cfl loop " + bc)
     s.close()
+
+
+# members with an open boundary: windows of 256 cells that own 182 (rk 3) or 206
+# (rk 2), one, two and more of them, a last one of a single cell, members smaller
+# than a window or of exactly one; ended by tend and by max_steps at each place in
+# a launch of up to four steps; with 800 more members, which end after two
+# steps, in stages before and in windows from then on
+@pytest.mark.parametrize("chunk,more", [(1, 0), (3, 0), (8, 0), (21, 0), (1, 800), (3, 800)])
+def test_1d_member_windows(gpu, chunk, more):
+    cases = [(5, 2, 3, "mlau", 0), (6, 1, 2, "roe", 1), (182, 2, 3, "mlau", 2), (183, 2, 3, "lhlld", 3),
+             (206, 2, 2, "hlld", 4), (207, 1, 2, "mlau", 5), (248, 2, 3, "mlau", 6), (249, 2, 3, "hlld", 7),
+             (365, 2, 3, "lhlld", 8), (413, 2, 2, "mlau", 9), (1093, 2, 3, "mlau", 0), (547, 2, 3, "mlau", 11)]
+    cases += [(16, 2, 3, "mlau", 2)] * more
+    ens = E.Ensemble(budget_bytes=1 << 28)
+    ids, ref = [], []
+    for k, (n, odr, rk, flux, most) in enumerate(cases):
+        f0, p = P.brio_wu(max(n, 16))
+        f0 = np.ascontiguousarray(f0[:, (max(n, 16) - n) // 2:][:, :n + 8])
+        f0[2] += 0.1 * f0[0] * np.sin(7 * np.arange(n + 8) / n)
+        f0[4] += 0.5 * f0[2] ** 2 / f0[0]
+        tend = 3.0 / n
+        m = E.member(f0, M.scheme(odr, rk, flux, 1), 1.0 / n, tend=tend, cfl=0.4, vfloor=1.0, gamma=p["gamma"],
+                     bx=p["bx"], max_steps=most)
+        ids.append(ens.add(f0, m))
+        if k and cases[k] == cases[k - 1]:
+            ref.append(ref[-1])
+            continue
+        g = f0.copy()
+        t, ns, _ = O.run_to_1d(g, p["bx"], 1.0 / n, 4, p["gamma"], O.scheme(odr, rk, flux, 1), tend, 0.4, 1.0,
+                              max_steps=most)
+        ref.append((g, t, ns))
+    ens.run_all(chunk=chunk)
+    for k, i in enumerate(ids):
+        _, t, _, ns = ens.status(i)
+        assert (t, ns) == ref[k][1:], (cases[k], t, ns, ref[k][1:])
+        assert_same(ens.download(i), ref[k][0], "1D member %s" % (cases[k],))
+    ens.close()
