@@ -35,7 +35,8 @@ typedef struct mlau_srv_times {
 } mlau_srv_times;
 
 /* Start a server with a device-memory budget; steps_per_round is how many
- * steps run between admission points (the latency/overhead trade-off). */
+ * steps run between admission points (the latency/overhead trade-off); while no
+ * request has joined, rounds shorter than 2 ms take more, up to 2 ms. */
 int mlau_srv_create(long long budget_bytes, int steps_per_round, mlau_server **out);
 /* Drain: finish every admitted and queued request, then stop the worker. */
 void mlau_srv_destroy(mlau_server *s);
