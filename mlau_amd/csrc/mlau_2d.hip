@@ -223,6 +223,18 @@ static void sweeps2d(Handle *h, const U2 &in, const W2 &w, const G2 &g)
     MLAU_LAUNCH(h, K_SWEEPS2D, (k_sweeps2d<ODR, FLUX, MIX, false>), gr, dim3(64), in, w, g, ch, px, nyb);
 }
 
+// Primitives and weights in one pass, which forms the neighbours' velocities
+// again, or in two: a small grid's pass is its launch and one cell's chain, a
+// large one's its bytes.  Walls, 8 steps, us, two passes and one: MUSCL + MLAU 64^2 583
+// and 546, 256^2 1002 and 957, 515x391 1505 and 1455, 1024^2 6261 and 6233, 1300^2
+// 10152 and 10193; WCNS4 + LHLLD 64^2 631 and 597, 1024^2 7914 and 7875, 1300^2 12509
+// and 12554, 2048^2 32554 and 32728; mixed 515x391 1359 and 1320, 1300^2 8574 and
+// 8595, 2048^2 22045 and 22191.  Tune bit 2: the other choice.
+static bool one_prim_pass(const Handle *h, const G2 &g)
+{
+  return ((long)g.nx * g.ny < (5L << 18)) != ((h->tune & 4) != 0);
+}
+
 template <int ODR, int FLUX, int MIX>
 static void stage2d(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const W2 &w, const G2 &g, double ra,
                     double rb, int adv)
@@ -230,7 +242,7 @@ static void stage2d(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const 
   const int nx = g.nx, ny = g.ny;
   dim3 b256(256);
   dim3 gcell(region_pieces(nx, ny));
-  if (!(h->tune & 4)) {  // separate prim and aux passes (faster on one large grid); tune bit 2: one fused pass
+  if (!one_prim_pass(h, g)) {
     MLAU_LAUNCH(h, K_PRIM2D, (k_prim2d<ODR>), gcell, b256, in, w, g, h->bc);
     if (h->s.ctw) MLAU_LAUNCH(h, K_AUX2D, (k_aux2d<1>), gcell, b256, in, w, g, h->bc);
     else MLAU_LAUNCH(h, K_AUX2D, (k_aux2d<0>), gcell, b256, in, w, g, h->bc);

@@ -38,6 +38,25 @@ def test_2d_march_lengths(gpu, ny, nx, walls):
     s.close()
 
 
+# walls: primitives and weights in one pass below 1310720 cells with ghosts, two
+# from there on
+@pytest.mark.parametrize("ctw", [0, 1])
+@pytest.mark.parametrize("ny,nx", [(5, 4), (31, 70), (1272, 1015), (1272, 1016)])
+def test_2d_wall_primitive_passes(gpu, ny, nx, ctw):
+    g, p = P.vortex_2d(max(nx, ny, 16), 4)
+    f0 = np.ascontiguousarray(g[:, :ny + 8, :nx + 8])
+    for n in range(8):
+        O.lib().oc_bc2d(O._p(f0[n]), nx + 8, ny + 8, 4, 4, int(n == 5), 0, int(n == 6), KHI_Y[n])
+    dt = 0.2 * p["dx"] / O.cfl_vmax_2d(f0, 4, p["gamma"], 1.0)
+    f_o = f0.copy()
+    O.step_2d(f_o, dt, p["dx"], p["dy"], 4, p["gamma"], O.scheme(2, 3, "mlau", ctw), dn=(0,) * 8, dny=KHI_Y)
+    s = M.Solver(f0, M.scheme(2, 3, "mlau", ctw, dnys=KHI_Y), p["dx"], p["dy"], gamma=p["gamma"])
+    s.set_dt(dt)
+    s.step(1)
+    assert_same(s.download(), f_o, "2D walls %dx%d" % (nx, ny))
+    s.close()
+
+
 # y- and z-sweep marches of 1 to 8 faces per lane; 1, 2 and 4 planes per thread
 # in the aux, edge and update kernels; the last of each cut short
 @pytest.mark.parametrize("nz,ny,nx", [(4, 5, 6), (30, 21, 25), (7, 120, 125), (63, 50, 70), (85, 96, 97),
