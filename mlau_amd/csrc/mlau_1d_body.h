@@ -370,7 +370,7 @@ __host__ __device__ __forceinline__ int win1_halo(int K, int rk)
 
 struct Lds1d {
   double q[7][kWin1];  // primitives ro, vx, vy, vz, by, bz, pr
-  int m[kWin1];        // supersonic
+  int m[kWin1];        // ratio_class of the squared Mach number
   double l[7][kWin1];  // left state of the face above each cell
   double f[7][kWin1];  // flux through the face below each cell, argument order
   double end[2][7];    // new ghosts of the open ends
@@ -490,7 +490,7 @@ __device__ __forceinline__ void step1d_body(const U1d &in, const U1d &out, const
       S.q[4][t] = u[5];
       S.q[5][t] = u[6];
       S.q[6][t] = pr;
-      S.m[t] = ratio_ge1(v2, quot_ieee(g.gamma * pr, u[0]));  // supersonic switch (mhd_fd4c_1d.c:155-166)
+      S.m[t] = ratio_class(v2, quot_ieee(g.gamma * pr, u[0]));  // supersonic switch (mhd_fd4c_1d.c:155-166)
     }
     __syncthreads();
     double vr[7], dv0 = 0.0;
@@ -504,7 +504,7 @@ __device__ __forceinline__ void step1d_body(const U1d &in, const U1d &out, const
         for (int v = 0; v < 7; v++) W.q[v][m] = S.q[v][p];
       }
       const int lo = t > 0 ? t - 1 : 0, hi = t < kWin1 - 1 ? t + 1 : kWin1 - 1;
-      const bool sup = S.m[lo] | S.m[t] | S.m[hi];
+      const bool sup = any_ge1(S.m[lo], S.m[t], S.m[hi]);
       double vl[7];
       recon_p<ODR, MIX>(W, sup, g.bx, g.gamma, vl, vr);
       dv0 = W.q[1][2] - W.q[1][1];

@@ -37,7 +37,7 @@ __device__ __forceinline__ void xsweep2d_inl_body(const U2 &u, const W2 &w, cons
   const long s = (long)j * nx + c;
   Stencil S;
   double cxs = 0.0;
-  bool sup = false;
+  int sup[3];
 #pragma unroll
   for (int m = 0; m < 5; m++) {
     Prim2 P = prim2d_point<ODR>(u, g, bc, c - 2 + m, j);
@@ -49,11 +49,11 @@ __device__ __forceinline__ void xsweep2d_inl_body(const U2 &u, const W2 &w, cons
     S.q[4][m] = P.cy;
     S.q[5][m] = P.bz;
     S.q[6][m] = P.pr;
-    if (m >= 1 && m <= 3) sup |= prim2d_sup(g, P);
+    if (m >= 1 && m <= 3) sup[m - 1] = prim2d_sup(g, P);
     if (m == 2) cxs = P.cx;
   }
   double vl[7], vr[7];
-  recon_p<ODR, MIX>(S, sup, cxs, g.gamma, vl, vr);
+  recon_p<ODR, MIX>(S, any_ge1(sup[0], sup[1], sup[2]), cxs, g.gamma, vl, vr);
   double p[5];
 #pragma unroll
   for (int m = 0; m < 5; m++) p[m] = S.q[4][m] * S.q[1][m];
@@ -124,7 +124,7 @@ __device__ __forceinline__ void ysweep2d_inl_body(const U2 &u, const W2 &w, cons
     W[4][m] = P.bz;
     W[5][m] = P.cx;
     W[6][m] = P.pr;
-    supb = (supb & ~(1u << m)) | ((prim2d_sup(g, P) ? 1u : 0u) << m);
+    supb = (supb & ~(1u << m)) | ((prim2d_sup(g, P) & 1u) << m);
   };
   // shock sensor dvx of window row m (row R): aux2d_body's expression
   auto dvx = [&](int R, int m) {
