@@ -184,10 +184,12 @@ inline int march_chunk(long pieces, int faces, long others, double tail, int mos
 // depend on the march length.  FP64 fuses nothing and always takes the short
 // copy; so do longest marches, whose kernels are compiled without the choice
 // (with it the 128^3 mixed sweeps took 1 % longer).
-// The FP32 LHLLD solver itself fuses otherwise in the kernels with the choice of
-// the sweeps that read primitive arrays, so these keep to longest marches.
+// The FP32 LHLLD solver and the contracted FP64 Roe solver themselves fuse otherwise in
+// the kernels with the choice of the sweeps that read primitive arrays, so
+// these keep to longest marches.
 template <int FLUX, int MIX>
-constexpr bool whole_march = MIX == MLAU_MIXED && FLUX == FLUX_LHLLD;
+constexpr bool whole_march =
+    (MIX == MLAU_MIXED && FLUX == FLUX_LHLLD) || (MIX == MLAU_MIXED_RECON && FLUX == FLUX_ROE);
 __device__ __forceinline__ bool march_mid(int ch, unsigned c, int most) { return (ch * c) % most != 0; }
 
 }  // namespace mlau
