@@ -1,9 +1,9 @@
 // mlau_1d.hip -- 1D ideal-MHD step on gfx950 (FP64).
 //
-// k_step1d runs one or more whole steps of 1D/SERIAL/shock/mhd_fd4c_1d.c:60-271 in
+// k_step1d runs one or more whole FP64 steps of 1D/SERIAL/shock/mhd_fd4c_1d.c:60-271 in
 // one launch (step1d_body): each block advances a window of cells with its own
 // halo, from u0 to u1 or back.  Very long grids, where the repeated halo cells
-// cost more than the launches, take a stage in two launches or one:
+// cost more than the launches, and the mixed forms take a stage in two launches or one:
 //   k_sweep1d   primitives (:121-131, formed per stencil point) + reconstruction
 //               + Riemann solver, one wavefront per 63 faces (left face
 //               states passed by shuffle)                                :137-207
@@ -57,12 +57,12 @@ __global__ __launch_bounds__(256) void k_update1d(U1d in, U1d ut, U1d out, W1d w
 }
 
 // K whole steps (step1d_body); block 0 advances the time.
-template <int ODR, int FLUX, int MIX, bool PER>
+template <int ODR, int FLUX, bool PER>
 __global__ __launch_bounds__(PER ? kWin1 : kWin1 + 64) void k_step1d(U1d in, U1d out, G1d g, StepInfo *info, int rk,
                                                                      int K)
 {
   __shared__ Lds1d S;
-  step1d_body<ODR, FLUX, MIX, PER>(in, out, g, info->dtdx, rk, K, blockIdx.x, threadIdx.x, S);
+  step1d_body<ODR, FLUX, PER>(in, out, g, info->dtdx, rk, K, blockIdx.x, threadIdx.x, S);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     for (int k = 0; k < K; k++) info->tim += info->dt;
     info->nstep += K;
@@ -180,20 +180,20 @@ static void step1d(Handle *h)
 // or two per stage -> 1, 2, 4 steps per launch: 1024 cells 843 -> 558, 527, 534 /
 // 1049 -> 673, 625, 597; 65536: 1178 -> 854, 805, 784 / 1704 -> 1247, 1179, 1162;
 // 262144: 2292 -> 2019, 1899, 2193 / 3540 -> 3015, 2884, 3922; 1048576: 6461 -> 6885, 6936,
-// 8170 / 11050 -> 10566, 11347, 14478.  0: separate stage launches, also for
-// FP32 Riemann solvers and the mixed Roe solver, whose multiply-adds the
-// compiler would fuse otherwise here (rounding differences of 1e-9 to 1e-8).
+// 8170 / 11050 -> 10566, 11347, 14478.  0: separate stage launches, also for the mixed
+// forms, whose multiply-adds the compiler would fuse otherwise here (rounding differences
+// of 1e-16 with FP64 solvers and of 1e-9 to 1e-8 with FP32 or Roe's, between grids on the two sides of
+// the line).
 static int steps_per_launch1d(const Handle *h, bool cfl_mode)
 {
-  if ((h->tune & 8) || h->g.nx > 393216) return 0;
-  if (h->s.precision == MLAU_MIXED || (h->s.precision == MLAU_MIXED_RECON && h->s.flux == FLUX_ROE)) return 0;
+  if ((h->tune & 8) || h->g.nx > 393216 || h->s.precision != MLAU_FP64) return 0;
   if (cfl_mode) return 1;  // the next dt needs the whole grid
   return h->g.nx > 131072 ? 2 : 4;
 }
 
 // Steps in launches of up to `most` whole steps, from one state to the other and
 // back; an odd number of launches ends with a copy into u0.
-template <int ODR, int FLUX, int MIX>
+template <int ODR, int FLUX>
 static void steps1d(Handle *h, int nsteps, int most, bool cfl_mode, double cfl, double vfloor)
 {
   U1d u0, u1;
@@ -210,9 +210,9 @@ static void steps1d(Handle *h, int nsteps, int most, bool cfl_mode, double cfl, 
     const dim3 gr((nx - 8 + own - 1) / own);
     const U1d &in = j & 1 ? u1 : u0, &out = j & 1 ? u0 : u1;
     if (open)
-      MLAU_LAUNCH(h, K_STEP1D, (k_step1d<ODR, FLUX, MIX, false>), gr, dim3(kWin1 + 64), in, out, g, h->info, rk, K);
+      MLAU_LAUNCH(h, K_STEP1D, (k_step1d<ODR, FLUX, false>), gr, dim3(kWin1 + 64), in, out, g, h->info, rk, K);
     else
-      MLAU_LAUNCH(h, K_STEP1D, (k_step1d<ODR, FLUX, MIX, true>), gr, dim3(kWin1), in, out, g, h->info, rk, K);
+      MLAU_LAUNCH(h, K_STEP1D, (k_step1d<ODR, FLUX, true>), gr, dim3(kWin1), in, out, g, h->info, rk, K);
     if (cfl_mode) check1d(h, out, g, cfl, vfloor);
   }
   if (m & 1) MLAU_LAUNCH(h, K_STEP1D, k_copy1d, dim3((nx + 255) / 256), dim3(256), u1, u0, nx);
@@ -240,20 +240,15 @@ static Step1Fn pick1(int flux, int precision)
   }
 }
 
-template <int ODR, int MIX>
-static Steps1Fn pick1sf(int flux)
+template <int ODR>
+static Steps1Fn pick1s(int flux)
 {
   switch (flux) {
-  case FLUX_MLAU: return steps1d<ODR, FLUX_MLAU, MIX>;
-  case FLUX_ROE: return steps1d<ODR, FLUX_ROE, MLAU_FP64>;  // FP64 only (steps_per_launch1d)
-  case FLUX_HLLD: return steps1d<ODR, FLUX_HLLD, MIX>;
-  default: return steps1d<ODR, FLUX_LHLLD, MIX>;
+  case FLUX_MLAU: return steps1d<ODR, FLUX_MLAU>;
+  case FLUX_ROE: return steps1d<ODR, FLUX_ROE>;
+  case FLUX_HLLD: return steps1d<ODR, FLUX_HLLD>;
+  default: return steps1d<ODR, FLUX_LHLLD>;
   }
-}
-template <int ODR>
-static Steps1Fn pick1s(int flux, int precision)
-{
-  return precision == MLAU_MIXED_RECON ? pick1sf<ODR, MLAU_MIXED_RECON>(flux) : pick1sf<ODR, MLAU_FP64>(flux);
 }
 
 int run_cfl_1d(Handle *h, double cfl, double vfloor)
@@ -272,10 +267,10 @@ int run_steps_1d(Handle *h, int nsteps, bool cfl_mode, double cfl, double vfloor
   if (const int most = steps_per_launch1d(h, cfl_mode)) {
     Steps1Fn fs;
     switch (h->s.odr) {
-    case 1: fs = pick1s<1>(h->s.flux, h->s.precision); break;
-    case 2: fs = pick1s<2>(h->s.flux, h->s.precision); break;
-    case 3: fs = pick1s<3>(h->s.flux, h->s.precision); break;
-    default: fs = pick1s<4>(h->s.flux, h->s.precision); break;
+    case 1: fs = pick1s<1>(h->s.flux); break;
+    case 2: fs = pick1s<2>(h->s.flux); break;
+    case 3: fs = pick1s<3>(h->s.flux); break;
+    default: fs = pick1s<4>(h->s.flux); break;
     }
     fs(h, nsteps, most, cfl_mode, cfl, vfloor);
     return (int)hipGetLastError();

@@ -345,7 +345,7 @@ __device__ __forceinline__ void stage1d_body(U1d in, U1d ut, U1d out, G1d g, dou
 }
 
 // ------------------------------------------------------------- whole steps
-// K steps in one launch.  A block holds a window of kWin1 cells, one per lane
+// K steps in one launch, FP64.  A block holds a window of kWin1 cells, one per lane
 // of its first four wavefronts, with the state in registers; primitives, left
 // states and fluxes pass between lanes through LDS.  Nothing crosses blocks:
 // each stage the outer cells of the window lose their meaning by the reach of
@@ -378,7 +378,7 @@ struct Lds1d {
 
 // Flux differences of cell a (4 <= a <= nx-5) straight from the arrays, ghosts as
 // they stand: what a stage of the separate kernels gives.
-template <int ODR, int FLUX, int MIX>
+template <int ODR, int FLUX>
 __device__ __forceinline__ void flux_diff1d(const U1d &in, const G1d &g, int a, double (&du)[7])
 {
   constexpr int lo = ODR <= 2 ? 0 : -1, hi = ODR <= 2 ? 1 : 2;  // faces a+lo..a+hi
@@ -409,9 +409,9 @@ __device__ __forceinline__ void flux_diff1d(const U1d &in, const G1d &g, int a, 
     }
     const bool sup = dmax(r[1], dmax(r[2], r[3])) >= 1.0;
     double vl[7], vr[7], f[7];
-    recon_p<ODR, MIX>(W, sup, g.bx, g.gamma, vl, vr);
+    recon<ODR>(W, sup, g.bx, g.gamma, vl, vr);
     if (j >= a + lo) {
-      riemann_p<FLUX, MIX>(L, vr, g.bx, g.gamma, W.q[1][2] - W.q[1][1], 0.0, f);
+      riemann<FLUX>(L, vr, g.bx, g.gamma, W.q[1][2] - W.q[1][1], 0.0, f);
       const double fa[7] = {f[0], f[1], f[2], f[3], f[6], f[4], f[5]};
 #pragma unroll
       for (int n = 0; n < 7; n++) {
@@ -429,7 +429,7 @@ __device__ __forceinline__ void flux_diff1d(const U1d &in, const G1d &g, int a, 
     du[n] = ODR <= 2 ? diff4<ODR>(0.0, F[2][n], F[3][n], 0.0) : diff4<ODR>(F[0][n], F[1][n], F[2][n], F[3][n]);
 }
 
-template <int ODR, int FLUX, int MIX, bool PER>
+template <int ODR, int FLUX, bool PER>
 __device__ __forceinline__ void step1d_body(const U1d &in, const U1d &out, const G1d &g, double dtdx, int rk, int K,
                                             unsigned b, unsigned tid, Lds1d &S)
 {
@@ -472,7 +472,7 @@ __device__ __forceinline__ void step1d_body(const U1d &in, const U1d &out, const
     }
     if (PER && raw && s == 0) {
       double du[7];
-      flux_diff1d<ODR, FLUX, MIX>(in, g, at, du);
+      flux_diff1d<ODR, FLUX>(in, g, at, du);
 #pragma unroll
       for (int n = 0; n < 7; n++) u[n] = 0.0 * ut[n] + 1.0 * (u[n] - dtdx * du[n]);
       continue;
@@ -506,7 +506,7 @@ __device__ __forceinline__ void step1d_body(const U1d &in, const U1d &out, const
       const int lo = t > 0 ? t - 1 : 0, hi = t < kWin1 - 1 ? t + 1 : kWin1 - 1;
       const bool sup = any_ge1(S.m[lo], S.m[t], S.m[hi]);
       double vl[7];
-      recon_p<ODR, MIX>(W, sup, g.bx, g.gamma, vl, vr);
+      recon<ODR>(W, sup, g.bx, g.gamma, vl, vr);
       dv0 = W.q[1][2] - W.q[1][1];
 #pragma unroll
       for (int k = 0; k < 7; k++) S.l[k][t] = vl[k];
@@ -539,7 +539,7 @@ __device__ __forceinline__ void step1d_body(const U1d &in, const U1d &out, const
       const int lo = t > 0 ? t - 1 : 0;
 #pragma unroll
       for (int k = 0; k < 7; k++) L[k] = S.l[k][lo];
-      riemann_p<FLUX, MIX>(L, vr, g.bx, g.gamma, dv0, 0.0, f);
+      riemann<FLUX>(L, vr, g.bx, g.gamma, dv0, 0.0, f);
       S.f[0][t] = f[0];
       S.f[1][t] = f[1];
       S.f[2][t] = f[2];

@@ -96,3 +96,46 @@ def test_3d_any_march(gpu, monkeypatch, nz, ny, nx, flux, precision):
         sch = M.scheme(odr, 3, flux, 1, precision=precision)
         a, b = [one_way(monkeypatch, t, f0, sch, (p["dx"], p["dy"], p["dz"]), p["gamma"], 5e-4) for t in (0, 64)]
         assert_same(a, b, "3D %dx%dx%d odr %d" % (nx, ny, nz, odr))
+
+
+def tube(n, copies):
+    """Waves in every field and a contact in each half of n cells, and the same with the middle
+    cell repeated over the length of copies - 1 more of them."""
+    x = np.arange(n + 8) / n
+    ro = 1.0 + 0.3 * np.sin(9 * x + 1) + 0.5 * ((x > 0.2) & (x < 0.8))
+    v = [0.4 * np.sin(5 * x), 0.3 * np.cos(7 * x), 0.2 * np.sin(4 * x + 2)]
+    by, bz, pr = 0.6 + 0.3 * np.cos(6 * x), 0.2 * np.sin(11 * x), 1.0 + 0.2 * np.cos(8 * x)
+    p = {"gamma": 5.0 / 3.0, "bx": 0.75}
+    en = pr / (p["gamma"] - 1) + 0.5 * (ro * sum(c * c for c in v) + p["bx"] ** 2 + by ** 2 + bz ** 2)
+    f = np.array([ro] + [ro * c for c in v] + [en, by, bz])
+    m = n // 2 + 4
+    return f, np.concatenate([f[:, :m]] + [f[:, m:m + 1]] * ((copies - 1) * n) + [f[:, m:]], axis=1), p
+
+
+# whole steps per launch up to 393216 cells in FP64, a launch or two per stage above: the
+# same cells in a short grid and in a long one, as far from the cut as the stencils
+# reach; periodic: ghosts from the other end, and ghosts filled otherwise
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64"] + MIXED)
+@pytest.mark.parametrize("flux", FLUXES)
+@pytest.mark.parametrize("n", [600, 1499])
+def test_1d_any_length(gpu, n, flux, precision):
+    short, long, p = tube(n, 400000 // n + 1)
+    for odr in (1, 2, 3, 4):
+        for rk, steps in ((1, 3), (2, 2), (3, 5)):
+            for bc in ("open", "periodic", "periodic, other ghosts"):
+                out = []
+                for f in (short, long):
+                    f0 = f.copy()
+                    if bc == "periodic":
+                        P.periodic_fill(f0)
+                    s = M.Solver(f0, M.scheme(odr, rk, flux, 1, precision=precision, bc1d=bc.split(",")[0]), 1.0 / n,
+                                 gamma=p["gamma"], bx=p["bx"])
+                    s.set_dt(0.05 / n)
+                    s.step(steps)
+                    out.append(s.download())
+                    s.close()
+                k = n // 2 - 4 * rk * steps
+                what = "odr %d rk %d %s" % (odr, rk, bc)
+                assert_same(out[0][:, :k], out[1][:, :k], what + ", low end")
+                assert_same(out[0][:, -k:], out[1][:, -k:], what + ", high end")
