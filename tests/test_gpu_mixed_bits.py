@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import mlau_amd as M
+from mlau_amd import ensemble as E
 from mlau_amd import problems as P
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -139,3 +140,47 @@ def test_1d_any_length(gpu, n, flux, precision):
                 what = "odr %d rk %d %s" % (odr, rk, bc)
                 assert_same(out[0][:, :k], out[1][:, :k], what + ", low end")
                 assert_same(out[0][:, -k:], out[1][:, -k:], what + ", high end")
+
+
+# members with an open boundary at odr <= 2: windows of whole steps while a group's
+# windows (running members of the mean size) fill the 256 CUs at most three times,
+# stage launches above.  Alone, beside a member of 3500 windows that runs as long, and
+# beside one of 870 that ends after two steps.
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64"] + MIXED)
+@pytest.mark.parametrize("flux", FLUXES)
+@pytest.mark.parametrize("odr,rk", [(1, 2), (1, 3), (2, 2), (2, 3)])
+def test_1d_members_in_windows_or_stages(gpu, odr, rk, flux, precision):
+    sch = M.scheme(odr, rk, flux, 1, precision=precision)
+    out = {}
+    for beside in ("alone", "long", "short"):
+        ens = E.Ensemble(budget_bytes=1 << 29)
+        ens.kernel_timing(True)
+        ids = []
+        for n, steps in ((5, 7), (183, 0), (700, 14)):
+            f, _, p = tube(n, 1)
+            m = E.member(f, sch, 1.0 / n, tend=4.0 / n, cfl=0.4, vfloor=1.0, gamma=p["gamma"], bx=p["bx"], max_steps=steps)
+            ids.append(ens.add(f, m))
+        if beside != "alone":
+            n = (870 if beside == "short" else 3500) * (182 if rk == 3 else 206)
+            f, _, p = tube(n, 1)
+            ens.add(f, E.member(f, sch, 1.0 / n, tend=1.0, cfl=0.4, vfloor=1.0, gamma=p["gamma"], bx=p["bx"],
+                                max_steps=2 if beside == "short" else 40))
+        steps = 0
+        while any(ens.status(i)[0] == E.RUNNING for i in ids):
+            ens.run(5)
+            steps += 5
+        st = {k: v[1] for k, v in ens.kernel_stats().items()}
+        sweeps, stages = st.get("ens_xsweep", 0), st.get("ens_stage", 0)
+        if beside == "alone":
+            assert sweeps == 0 and stages > 0, st
+        elif beside == "long":
+            assert sweeps == steps and stages == steps * (rk - 1), st
+        else:
+            assert sweeps == 5 and stages > 5 * (rk - 1), st
+        out[beside] = [ens.download(i) for i in ids], [ens.status(i) for i in ids]
+        ens.close()
+    for beside in ("long", "short"):
+        assert out[beside][1] == out["alone"][1], beside
+        for a, b in zip(out[beside][0], out["alone"][0]):
+            assert_same(a, b, "member, companion %s" % beside)
