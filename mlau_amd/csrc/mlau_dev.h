@@ -51,7 +51,9 @@ MLAU_DEV double rcp_ieee(double d)
   return __builtin_amdgcn_div_fixup(y, d, 1.0);
 }
 // n / d where |d| is as above, |n| is zero or above 2^-968 (so that no residual
-// underflows) and the quotient is zero or normal.
+// underflows) and the quotient is zero, normal or beyond the largest double: there n * y
+// is infinite and its correction NaN, which the minimum turns back (v_div_fixup sets the
+// sign and settles NaN operands, 0 / 0 and infinite ones).
 MLAU_DEV double quot_ieee(double n, double d)
 {
   double y = __builtin_amdgcn_rcp(d);
@@ -59,7 +61,7 @@ MLAU_DEV double quot_ieee(double n, double d)
   y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
   double q = n * y;
   q = __builtin_fma(__builtin_fma(-d, q, n), y, q);
-  return __builtin_amdgcn_div_fixup(q, d, n);
+  return __builtin_amdgcn_div_fixup(__builtin_fmin(q, __builtin_huge_val()), d, n);
 }
 // sqrt(x) for x above 2^-767, zeros, infinities and NaN.
 MLAU_DEV double sqrt_ieee(double x)
