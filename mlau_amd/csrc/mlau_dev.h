@@ -75,22 +75,22 @@ MLAU_DEV double sqrt_ieee(double x)
   s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
   return __builtin_amdgcn_class(x, 0x260) ? x : s;  // -0, +0, +inf
 }
-// For a >= 0: 1 where a / b >= 1, 2 where it is NaN, else 0.  A quotient of doubles
-// below 1 is at most 1 - 2^-53 and rounds to it, so for positive finite b the
-// division is not needed.
+// For a >= 0, and b NaN where a is: 1 where a / b >= 1, 2 where it is NaN, else 0.  A
+// quotient of doubles below 1 is at most 1 - 2^-53 and rounds to it, so for positive
+// finite b the division is not needed.
 MLAU_DEV int ratio_class(double a, double b)
 {
   if (__builtin_expect(!(b > 0.0 && b < __builtin_huge_val()), 0)) {
     const double q = a / b;
     return q >= 1.0 ? 1 : (q != q ? 2 : 0);
   }
-  return a >= b ? 1 : (a != a ? 2 : 0);
+  return a >= b;
 }
 MLAU_DEV bool ratio_ge1(double a, double b) { return ratio_class(a, b) == 1; }
 // dmax(m[0], dmax(m[1], m[2])) >= 1 by the classes of the three: dmax gives its
 // second argument where either is NaN, so the last one's NaN (a cold cell at rest,
 // 0 / 0) decides and the others' do not count.
-MLAU_DEV bool any_ge1(int c0, int c1, int c2) { return ((c0 | c1 | c2) & 1) && c2 != 2; }
+MLAU_DEV bool any_ge1(int c0, int c1, int c2) { return (((c0 | c1) & 1) | c2) == 1; }
 
 // include/interp.h:30-37
 MLAU_DEV void muscl_mm(double f1, double f2, double f3, double &fl, double &fr)
