@@ -69,6 +69,20 @@ double seconds_since(std::chrono::steady_clock::time_point t0)
   return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
 
+// Steps of the round after one of `last` steps that took `seconds`, for the same members:
+// as many as fit in kRoundS, at most four times the last at once and `least` at
+// least.  A round costs the host about 200 us whatever it holds, and the tail of a served burst is
+// often 1D requests alone, whose steps take 13 us: a tube of 5000 cells to its end time, at 31 us
+// a step, took 261 ms in rounds of 4 steps, 173 so.  Rounded down, so that the
+// next round stays there, to whole graphs: eight steps, 32 of 1D windows.
+int next_round(int least, int last, double seconds)
+{
+  constexpr double kRoundS = 2e-3;
+  if (last == 0 || !(seconds > 0.0)) return least;
+  const int n = (int)std::min(4.0 * last, kRoundS / seconds * last);
+  return std::max(least, n >= 64 ? n / 32 * 32 : n >= 8 ? n / 8 * 8 : n);
+}
+
 }  // namespace
 
 using mlau::fail;
@@ -91,6 +105,7 @@ struct mlau_server {
     {
       std::lock_guard<std::mutex> lk(s->mu);
       s->round_done = true;
+      s->ended = std::chrono::steady_clock::now();
     }
     s->cv_work.notify_all();
   }
@@ -98,7 +113,8 @@ struct mlau_server {
   long long budget = 0;
   int steps = 8;             // steps of a round after an admission, the least of any round
   int round_n = 0;           // steps and seconds of the last round
-  double round_s = 0.0;
+  double round_s = 0.0;      // (from the launch to the end of the steps: host copies beside them don't count)
+  std::chrono::steady_clock::time_point ended;  // end of the round's steps
   bool admitted = false;     // members joined since the last round was queued
   double hold_s = 1.0;            // a head request waiting longer than this blocks backfill
   std::chrono::steady_clock::time_point t0;
@@ -236,21 +252,13 @@ struct mlau_server {
     }
   }
 
-  // Steps of the next round: `steps`, or as many as take kRoundS where the last
-  // round was shorter and its members are the ones still running.  A round costs
-  // the host about 200 us whatever it holds, and the tail of a served burst is
-  // often 1D requests alone, whose steps take 31 us: a tube of 5000 cells to its
-  // end time took 261 ms in rounds of 4 steps, 173 so.  An admission sets the round
-  // back to `steps`, since a new member may make the steps longer.
+  // Steps of the next round: an admission sets it back to `steps`, since a new
+  // member may make the steps longer.
   int round_steps()
   {
-    constexpr double kRoundS = 2e-3;
     const bool fresh = admitted;
     admitted = false;
-    if (fresh || round_n == 0 || !(round_s > 0.0) || round_s >= kRoundS) return steps;
-    // at most four times the last round at once; whole graphs of eight steps
-    const int n = (int)std::min(4.0 * round_n, kRoundS / round_s * round_n);
-    return n <= steps ? steps : std::max(steps, (n + 7) / 8 * 8);
+    return fresh ? steps : next_round(steps, round_n, round_s);
   }
 
   void run()
@@ -304,6 +312,7 @@ struct mlau_server {
       {
         std::lock_guard<std::mutex> lk(mu);
         round_done = false;
+        ended = began;
       }
       if (mlau_ens_on_ready(ens, &mlau_server::round_end, this)) {
         std::lock_guard<std::mutex> lk(mu);
@@ -323,8 +332,9 @@ struct mlau_server {
       }
       int nrun = 0;
       if (mlau_ens_sync(ens, &nrun)) fail_running(mlau_last_error());
+      std::lock_guard<std::mutex> lk(mu);
       round_n = n;
-      round_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - began).count();
+      round_s = std::chrono::duration<double>(ended - began).count();  // 0 without a notice: `steps` again
     }
     if (ens) mlau_ens_destroy(ens);
     ens = nullptr;
