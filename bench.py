@@ -743,7 +743,9 @@ def main():
     # algorithmic bytes of each kernel per launch: the arrays it must read and
     # write once per interior cell, 8 B each (update2d: 21 + 8 in the first RK
     # stage, which reads no step-start state, 29 + 8 in the other two)
-    kern_arrays = {"ysweep2d_inl": 8 + 9, "xsweep2d_inl": 8 + 8, "ysweep2d": 11 + 8, "xsweep2d": 11 + 8,
+    # the sweeps of a stage are one launch (periodic grids: the state read, both sweeps' fluxes
+    # written), or two with MLAU_TUNE bit 6
+    kern_arrays = {"sweeps2d": 8 + 17, "ysweep2d_inl": 8 + 9, "xsweep2d_inl": 8 + 8, "ysweep2d": 11 + 8, "xsweep2d": 11 + 8,
                    "update2d": (29 + 37 + 37) / 3.0, "prim2d": 8 + 7, "aux2d": 5 + 3, "primaux2d": 8 + 10,
                    "ez2d": 5 + 1, "cfl2d": 8, "bc2d": 0}
     dom = max(stats.items(), key=lambda kv: kv[1][0])

@@ -1,12 +1,13 @@
 // mlau_2d.hip -- 2D ideal-MHD + CT step on gfx950 (FP64).
 //
-// One RK stage (2D/SERIAL/OTvortex/mhd_fd_ct_2d.c:165-639) is six kernels:
+// One RK stage (2D/SERIAL/OTvortex/mhd_fd_ct_2d.c:165-639) is five kernels:
 //   k_prim2d    face B -> centre (cx,cy) and primitives (vx,vy,vz,pr,m2)   :172-223
 //   k_aux2d     CT upwind weight ctx and shock sensors dvx,dvy            :224-271
-//   k_xsweep2d  X reconstruction + Riemann solver, one wavefront per 63
+//   k_sweeps2d  both sweeps, by blocks:
+//     x         reconstruction + Riemann solver, one wavefront per 63
 //               faces of a row; each lane reconstructs one cell and hands
 //               its left face state to the next lane by a wave shuffle    :273-362
-//   k_ysweep2d  Y reconstruction + Riemann solver, one lane per column
+//     y         reconstruction + Riemann solver, one lane per column
 //               marching up a chunk of rows with the 5-row stencil held in
 //               registers (coalesced rows, no reconstruction twice)      :404-493
 //   k_ez2d      corner E-field from both sweeps' induction fluxes       :364-402,495-533
@@ -50,21 +51,6 @@ __global__ __launch_bounds__(256) void k_primaux2d(U2 u, W2 w, G2 g, BcFlags bc)
   primaux2d_body<ODR, CTW>(u, w, g, bc, i, j);
 }
 
-// x sweep: row-flattened wavefronts, 4 per block
-template <int ODR, int FLUX, int MIX>
-__global__ __launch_bounds__(256) void k_xsweep2d(U2 u, W2 w, G2 g)
-{
-  const long W = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (W >= xsweep_waves(g.ny, g.nx)) return;  // whole wavefront
-  xsweep2d_body<ODR, FLUX, MIX>(u, w, g, W, threadIdx.x & 63);
-}
-
-template <int ODR, int FLUX, int MIX>
-__global__ __launch_bounds__(64) void k_ysweep2d(U2 u, W2 w, G2 g, int ch)
-{
-  ysweep2d_body<ODR, FLUX, MIX, false>(u, w, g, ch, false, blockIdx.x, blockIdx.y, threadIdx.x);
-}
-
 template <int ODR>
 __global__ __launch_bounds__(256) void k_ez2d(W2 w, G2 g)
 {
@@ -91,29 +77,14 @@ __global__ __launch_bounds__(256) void k_update2d_per(U2 in, U2 ut, U2 out, W2 w
   update2d_body<ODR, FIRST, true>(in, ut, out, w, g, info->dtdx, info->dtdy, ra, rb, i, j);
 }
 
-// Periodic grids: the sweeps and the E-field form primitives, shock sensors
-// and CT weights from the state themselves (mlau_2d_fused.h).
-template <int ODR, int FLUX, int MIX>
-__global__ __launch_bounds__(256) void k_xsweep2d_inl(U2 u, W2 w, G2 g)
-{
-  const long W = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (W >= xsweep_waves(g.ny, g.nx)) return;  // whole wavefront
-  xsweep2d_inl_body<ODR, FLUX, MIX>(u, w, g, W, threadIdx.x & 63);
-}
-
-template <int ODR, int FLUX, int MIX, int CTW>
-__global__ __launch_bounds__(64) void k_ysweep2d_inl(U2 u, W2 w, G2 g, int ch)
-{
-  ysweep2d_inl_body<ODR, FLUX, MIX, CTW, false>(u, w, g, ch, false, blockIdx.x, blockIdx.y, threadIdx.x);
-}
-
-// Both sweeps in one launch, as all stages run them: blocks below `ny` are
-// y-sweep blocks (px pieces of a row by marches), the others one x-sweep
-// wavefront each.  The sweeps share no output, and both fit two wavefronts to
+// Both sweeps in one launch: blocks below `ny` are y-sweep blocks (px pieces of a row
+// by marches), the others one x-sweep wavefront each (row-flattened).  The sweeps share no output, and both fit two wavefronts to
 // a SIMD.  Against two launches on two streams, where a fork and a join
 // wait on each other's events, 8 steps, us: 64^2 964 -> 599, 256^2 1278 -> 1041,
 // 1024^2 6898 -> 6604, 2048^2 26117 -> 25610; mixed 256^2 1133 -> 826, 1024^2 5587 ->
 // 4797 (the x sweep's third wavefront lost nothing); walls 512^2 1991 -> 1825.
+// Periodic grids: primitives, shock sensors and CT weights from the state
+// itself (mlau_2d_fused.h).
 template <int ODR, int FLUX, int MIX, int CTW, bool SPLIT>
 __global__ __launch_bounds__(64) void k_sweeps2d_inl(U2 u, W2 w, G2 g, int ch, unsigned px, unsigned ny)
 {
@@ -199,28 +170,35 @@ static int ychunk(const Handle *h, const G2 &g)
                               h->s.precision != MLAU_FP64);
 }
 
-// Per-kernel timing and tune bit 6 launch the sweeps one by one.
-static bool one_by_one(const Handle *h) { return h->timing.enabled || (h->tune & 64); }
+// Launches of both sweeps: `go` takes the kernel id, the grid, whether marches are split,
+// their length and the number of y blocks.  Tune bit 6, for profiles of each sweep: one
+// after the other, each as its part of the joint launch's blocks, the mixed forms in longest
+// marches (same bits, march_mid).
+template <int MIX, typename Go>
+static void launch_sweeps2d(Handle *h, const G2 &g, int ch, int kx, int ky, Go go)
+{
+  const bool one_by_one = (h->tune & 64) != 0;
+  if (one_by_one && split_march<MIX>(ch)) ch = kMarch;
+  const unsigned px = (g.nx + 63) / 64, nyb = px * ((g.ny - 5 + ch - 1) / ch);
+  const unsigned xw = (unsigned)xsweep_waves(g.ny, g.nx);
+  if (one_by_one) {
+    go(kx, dim3(xw), false, ch, px, 0u);
+    go(ky, dim3(nyb), false, ch, px, nyb);
+  } else {
+    go(K_SWEEPS2D, dim3(nyb + xw), split_march<MIX>(ch), ch, px, nyb);
+  }
+}
 
 template <int ODR, int FLUX, int MIX>
 static void sweeps2d(Handle *h, const U2 &in, const W2 &w, const G2 &g)
 {
-  const unsigned px = (g.nx + 63) / 64;
-  const long xw = xsweep_waves(g.ny, g.nx);
-  int ch = whole_march<FLUX, MIX> ? kMarch : ychunk(h, g);
-  if (one_by_one(h)) {
-    if (split_march<MIX>(ch)) ch = kMarch;
-    MLAU_LAUNCH(h, K_XSWEEP2D, (k_xsweep2d<ODR, FLUX, MIX>), dim3((unsigned)((xw + 3) / 4)), dim3(256), in, w, g);
-    MLAU_LAUNCH(h, K_YSWEEP2D, (k_ysweep2d<ODR, FLUX, MIX>), dim3(px, (g.ny - 5 + ch - 1) / ch), dim3(64), in, w, g,
-                ch);
-    return;
-  }
-  const unsigned nyb = px * ((g.ny - 5 + ch - 1) / ch);
-  const dim3 gr(nyb + (unsigned)xw);
-  if (split_march<MIX>(ch))
-    MLAU_LAUNCH(h, K_SWEEPS2D, (k_sweeps2d<ODR, FLUX, MIX, MIX != MLAU_FP64>), gr, dim3(64), in, w, g, ch, px, nyb);
-  else
-    MLAU_LAUNCH(h, K_SWEEPS2D, (k_sweeps2d<ODR, FLUX, MIX, false>), gr, dim3(64), in, w, g, ch, px, nyb);
+  const int ch = whole_march<FLUX, MIX> ? kMarch : ychunk(h, g);
+  launch_sweeps2d<MIX>(h, g, ch, K_XSWEEP2D, K_YSWEEP2D, [&](int k, dim3 gr, bool split, int c, unsigned px, unsigned nyb) {
+    if (split)
+      MLAU_LAUNCH(h, k, (k_sweeps2d<ODR, FLUX, MIX, MIX != MLAU_FP64>), gr, dim3(64), in, w, g, c, px, nyb);
+    else
+      MLAU_LAUNCH(h, k, (k_sweeps2d<ODR, FLUX, MIX, false>), gr, dim3(64), in, w, g, c, px, nyb);
+  });
 }
 
 // Primitives and weights in one pass, which forms the neighbours' velocities
@@ -271,23 +249,13 @@ static void stage2d(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const 
 template <int ODR, int FLUX, int MIX, int CTW>
 static void sweeps2d_inl(Handle *h, const U2 &in, const W2 &w, const G2 &g)
 {
-  const unsigned px = (g.nx + 63) / 64;
-  const long xw = xsweep_waves(g.ny, g.nx);
-  int ch = ychunk(h, g);
-  if (one_by_one(h)) {
-    if (split_march<MIX>(ch)) ch = kMarch;
-    MLAU_LAUNCH(h, K_XSW2D_INL, (k_xsweep2d_inl<ODR, FLUX, MIX>), dim3((unsigned)((xw + 3) / 4)), dim3(256), in, w, g);
-    MLAU_LAUNCH(h, K_YSW2D_INL, (k_ysweep2d_inl<ODR, FLUX, MIX, CTW>), dim3(px, (g.ny - 5 + ch - 1) / ch), dim3(64),
-                in, w, g, ch);
-    return;
-  }
-  const unsigned nyb = px * ((g.ny - 5 + ch - 1) / ch);
-  const dim3 gr(nyb + (unsigned)xw);
-  if (split_march<MIX>(ch))
-    MLAU_LAUNCH(h, K_SWEEPS2D, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, MIX != MLAU_FP64>), gr, dim3(64), in, w, g, ch, px,
-                nyb);
-  else
-    MLAU_LAUNCH(h, K_SWEEPS2D, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, false>), gr, dim3(64), in, w, g, ch, px, nyb);
+  launch_sweeps2d<MIX>(h, g, ychunk(h, g), K_XSW2D_INL, K_YSW2D_INL,
+                       [&](int k, dim3 gr, bool split, int c, unsigned px, unsigned nyb) {
+    if (split)
+      MLAU_LAUNCH(h, k, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, MIX != MLAU_FP64>), gr, dim3(64), in, w, g, c, px, nyb);
+    else
+      MLAU_LAUNCH(h, k, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, false>), gr, dim3(64), in, w, g, c, px, nyb);
+  });
 }
 
 // Periodic grids (with room for the ghost images written by the update): the

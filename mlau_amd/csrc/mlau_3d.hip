@@ -3,10 +3,11 @@
 // One RK stage of 3D/MPI/OTvortex/mhd_fd_ct_3d.c:178-1176:
 //   k_prim3d    face B -> centre (cx,cy,cz) + primitives, halo fills folded in   :186-262
 //   k_aux3d_zm  CT weights ct0 (xy), ct1 (yz), ct2 (zx) and shock sensors,
-//               a thread per column walking 8 cells along z                    :264-377
-//   k_xsweep3d  X reconstruction + Riemann, one wavefront per 63 faces of a row  :379-493
-//   k_msweep3d  Y and Z reconstruction + Riemann: one lane per x, marching a
-//               chunk along y (or z) with the stencil in registers            :587-701,795-909
+//               a thread per column walking 1 to 8 cells along z                    :264-377
+//   k_sweeps3d  all sweeps, by blocks:
+//     x         reconstruction + Riemann, one wavefront per 63 faces of a row    :379-493
+//     y, z      reconstruction + Riemann: one lane per x, marching a chunk along
+//               y (or z) with the stencil in registers                       :587-701,795-909
 //   k_edge3d    edge E-fields ex,ey,ez from the three sweeps                   :494-585,702-793,910-1001
 //   k_update3d  cell update, CT Bx/By/Bz, SSP-RK combine                       :1003-1157
 //   k_bc3d      ghost cells (single-rank periodic copies / walls)               :1161-1175
@@ -62,18 +63,9 @@ __global__ __launch_bounds__(256) void k_aux3d_zm(int cz, U3 u, const double *vx
   aux3d_zm_body<CTW>(cz, u, vx, vy, vz, ct0, ct1, ct2, dvx, dvy, dvz, g, bc, i, j, b.plane);
 }
 
-// x sweep: row-flattened wavefronts, 4 per block
-template <int ODR, int FLUX, int MIX>
-__global__ __launch_bounds__(256) void k_xsweep3d(Sw3 w, G3 g)
-{
-  const long W = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (W >= xsweep_waves((long)g.ny * g.nz, g.nx)) return;  // whole wavefront
-  xsweep3d_body<ODR, FLUX, MIX>(w, g, W, threadIdx.x & 63);
-}
-
-// All three sweeps in one launch, as all stages run them: blocks below yb march
-// along y, those below yb + zb along z, the others are one x-sweep wavefront
-// each.  Against three launches on three streams with their fork and join, 8 steps, us:
+// All three sweeps in one launch: blocks below yb march along y, those below yb + zb
+// along z (lanes over the flattened columns of i and the third coordinate), the others
+// are one x-sweep wavefront each.  Against three launches on three streams with their fork and join, 8 steps, us:
 // 24^3 1654 -> 1081, 48^3 2823 -> 2352, 96^3 11773 -> 11463, 128^3 26804 -> 26623;
 // mixed 32^3 1766 -> 1180, 128^3 21044 -> 20492.
 template <int ODR, int FLUX, int MIX, bool SPLIT>
@@ -96,19 +88,6 @@ __global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_sweeps3d(Sw3 wx, Sw3 wy, 
   } else {
     xsweep3d_body<ODR, FLUX, MIX>(wx, g, (long)(b - yb - zb), threadIdx.x);
   }
-}
-
-// y/z sweeps: lanes over the flattened (i, third coordinate) columns; blocks
-// are (column piece, chunk along the sweep axis)
-template <int ODR, int FLUX, int AX, int MIX>
-__global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_msweep3d(Sw3 w, G3 g, int ch)
-{
-  const long nc = (AX == 1) ? g.nz : g.ny;
-  const unsigned pieces = (unsigned)((g.nx * nc + 63) / 64);
-  const long p = (long)(blockIdx.x % pieces) * 64 + threadIdx.x;
-  if (p >= g.nx * nc) return;
-  const unsigned c = blockIdx.x / pieces;
-  msweep3d_body<ODR, FLUX, AX, MIX, false>(w, g, ch, false, (int)(p % g.nx), c, (int)(p / g.nx));
 }
 
 template <int ODR>
@@ -250,21 +229,25 @@ static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double
   const int chy = whole ? kMarch : march_chunk(yw, ny - 5, xw + zw * nz, 0.2, kMarch, MIX != MLAU_FP64);
   const int chz = whole ? kMarch : march_chunk(zw, nz - 5, xw + yw * ny, 0.2, kMarch, MIX != MLAU_FP64);
   const Sw3 wx = sweep_view(h, in, 0), wy = sweep_view(h, in, 1), wz = sweep_view(h, in, 2);
-  if (h->timing.enabled || (h->tune & 64)) {  // per-kernel timing and tune bit 6: one by one
-    const int cy = MIX != MLAU_FP64 ? kMarch : chy, cz_ = MIX != MLAU_FP64 ? kMarch : chz;
-    MLAU_LAUNCH(h, K_XSWEEP3D, (k_xsweep3d<ODR, FLUX, MIX>), dim3((unsigned)((xw + 3) / 4)), b256, wx, g);
-    MLAU_LAUNCH(h, K_YSWEEP3D, (k_msweep3d<ODR, FLUX, 1, MIX>), dim3((unsigned)(yw * ((ny - 5 + cy - 1) / cy))),
-                dim3(64), wy, g, cy);
-    MLAU_LAUNCH(h, K_ZSWEEP3D, (k_msweep3d<ODR, FLUX, 2, MIX>), dim3((unsigned)(zw * ((nz - 5 + cz_ - 1) / cz_))),
-                dim3(64), wz, g, cz_);
-  } else {
-    const unsigned yb = (unsigned)(yw * ((ny - 5 + chy - 1) / chy)), zb = (unsigned)(zw * ((nz - 5 + chz - 1) / chz));
-    const dim3 gr(yb + zb + (unsigned)xw);
-    if (MIX != MLAU_FP64 && (chy < kMarch || chz < kMarch))
-      MLAU_LAUNCH(h, K_SWEEPS3D, (k_sweeps3d<ODR, FLUX, MIX, MIX != MLAU_FP64>), gr, dim3(64), wx, wy, wz, g, chy, chz,
-                  yb, zb);
+  const bool one_by_one = (h->tune & 64) != 0;
+  const bool split = MIX != MLAU_FP64 && !one_by_one && (chy < kMarch || chz < kMarch);
+  const int cy = one_by_one && MIX != MLAU_FP64 ? kMarch : chy, cz_ = one_by_one && MIX != MLAU_FP64 ? kMarch : chz;
+  const unsigned yb = (unsigned)(yw * ((ny - 5 + cy - 1) / cy)), zb = (unsigned)(zw * ((nz - 5 + cz_ - 1) / cz_));
+  auto sweeps = [&](int k, unsigned blocks, unsigned y, unsigned z) {
+    if (split)
+      MLAU_LAUNCH(h, k, (k_sweeps3d<ODR, FLUX, MIX, MIX != MLAU_FP64>), dim3(blocks), dim3(64), wx, wy, wz, g, cy, cz_,
+                  y, z);
     else
-      MLAU_LAUNCH(h, K_SWEEPS3D, (k_sweeps3d<ODR, FLUX, MIX, false>), gr, dim3(64), wx, wy, wz, g, chy, chz, yb, zb);
+      MLAU_LAUNCH(h, k, (k_sweeps3d<ODR, FLUX, MIX, false>), dim3(blocks), dim3(64), wx, wy, wz, g, cy, cz_, y, z);
+  };
+  // Tune bit 6, for profiles of each sweep: one after the other, each as its part of the
+  // joint launch's blocks, the mixed forms in longest marches (same bits, march_mid).
+  if (one_by_one) {
+    sweeps(K_XSWEEP3D, (unsigned)xw, 0, 0);
+    sweeps(K_YSWEEP3D, yb, yb, 0);
+    sweeps(K_ZSWEEP3D, zb, 0, zb);
+  } else {
+    sweeps(K_SWEEPS3D, yb + zb + (unsigned)xw, yb, zb);
   }
   Edge3 e;
   e.fxt = h->fx[4]; e.fxu = h->fx[5]; e.fcx0 = h->fcx[0]; e.fcx1 = h->fcx[1];
