@@ -86,7 +86,8 @@ __global__ __launch_bounds__(256) void k_update2d_per(U2 in, U2 ut, U2 out, W2 w
 // Periodic grids: primitives, shock sensors and CT weights from the state
 // itself (mlau_2d_fused.h).
 template <int ODR, int FLUX, int MIX, int CTW, bool SPLIT>
-__global__ __launch_bounds__(64) void k_sweeps2d_inl(U2 u, W2 w, G2 g, int ch, unsigned px, unsigned ny)
+__device__ __forceinline__ void sweeps2d_inl_body(const U2 &u, const W2 &w, const G2 &g, int ch, unsigned px,
+                                                  unsigned ny)
 {
   const unsigned b = blockIdx.x;
   if (b < ny)
@@ -95,8 +96,19 @@ __global__ __launch_bounds__(64) void k_sweeps2d_inl(U2 u, W2 w, G2 g, int ch, u
   else
     xsweep2d_inl_body<ODR, FLUX, MIX>(u, w, g, (long)(b - ny), threadIdx.x);
 }
+template <int ODR, int FLUX, int MIX, int CTW, bool SPLIT>
+__global__ __launch_bounds__(64) void k_sweeps2d_inl(U2 u, W2 w, G2 g, int ch, unsigned px, unsigned ny)
+{
+  sweeps2d_inl_body<ODR, FLUX, MIX, CTW, SPLIT>(u, w, g, ch, px, ny);
+}
+template <int ODR, int FLUX, int MIX, int CTW, bool SPLIT>
+__global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_sweeps2d_inl_two(U2 u, W2 w, G2 g, int ch, unsigned px,
+                                                                        unsigned ny)
+{
+  sweeps2d_inl_body<ODR, FLUX, MIX, CTW, SPLIT>(u, w, g, ch, px, ny);
+}
 template <int ODR, int FLUX, int MIX, bool SPLIT>
-__global__ __launch_bounds__(64) void k_sweeps2d(U2 u, W2 w, G2 g, int ch, unsigned px, unsigned ny)
+__device__ __forceinline__ void sweeps2d_body(const U2 &u, const W2 &w, const G2 &g, int ch, unsigned px, unsigned ny)
 {
   const unsigned b = blockIdx.x;
   if (b < ny)
@@ -104,6 +116,29 @@ __global__ __launch_bounds__(64) void k_sweeps2d(U2 u, W2 w, G2 g, int ch, unsig
   else
     xsweep2d_body<ODR, FLUX, MIX>(u, w, g, (long)(b - ny), threadIdx.x);
 }
+template <int ODR, int FLUX, int MIX, bool SPLIT>
+__global__ __launch_bounds__(64) void k_sweeps2d(U2 u, W2 w, G2 g, int ch, unsigned px, unsigned ny)
+{
+  sweeps2d_body<ODR, FLUX, MIX, SPLIT>(u, w, g, ch, px, ny);
+}
+template <int ODR, int FLUX, int MIX, bool SPLIT>
+__global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_sweeps2d_two(U2 u, W2 w, G2 g, int ch, unsigned px, unsigned ny)
+{
+  sweeps2d_body<ODR, FLUX, MIX, SPLIT>(u, w, g, ch, px, ny);
+}
+
+// Forms whose joint sweeps take 258 to 272 VGPRs by themselves, and so one wavefront a SIMD.
+// Launches of more wavefronts than two for each of the chip's 1024 SIMDs hold them to 256,
+// where 0 to 68 bytes are spilled; smaller ones gain nothing by it. us a step: walls, MUSCL + MLAU 64^2
+// 65.2 and 67.2, 515^2 237 and 218, 1400^2 1447 and 1239; WCNS4 + LHLLD 256^2 144 and 147, 900^2 739 and 662, 2048^2
+// 4015 and 3486; periodic, WCNS4 + MLAU 100^2 73.9 and 75.7, 256^2 141 and 135, 2048^2 4085 and 3299, Roe
+// 3963 and 3266. On the others the limit is not needed (WCNS3 + MLAU periodic 2048^2 2897 and 3104).
+template <int ODR, int FLUX, int MIX>
+constexpr bool two_waves_inl = MIX == MLAU_FP64 && ODR == 4 && (FLUX == FLUX_MLAU || FLUX == FLUX_ROE);
+template <int ODR, int FLUX, int MIX>
+constexpr bool two_waves = (MIX == MLAU_FP64 && ((FLUX == FLUX_MLAU && ODR >= 2) || (FLUX == FLUX_LHLLD && ODR == 4))) ||
+                           (MIX == MLAU_MIXED_RECON && FLUX == FLUX_MLAU && ODR == 4);
+constexpr unsigned kTwoWaves = 2048;
 
 // CT weight 1/2 at corners 3..nx-3 x 3..ny-3 (no upwind weighting)
 __global__ __launch_bounds__(256) void k_ctx_half2d(W2 w, G2 g)
@@ -194,10 +229,19 @@ static void sweeps2d(Handle *h, const U2 &in, const W2 &w, const G2 &g)
 {
   const int ch = whole_march<FLUX, MIX> ? kMarch : ychunk(h, g);
   launch_sweeps2d<MIX>(h, g, ch, K_XSWEEP2D, K_YSWEEP2D, [&](int k, dim3 gr, bool split, int c, unsigned px, unsigned nyb) {
-    if (split)
-      MLAU_LAUNCH(h, k, (k_sweeps2d<ODR, FLUX, MIX, MIX != MLAU_FP64>), gr, dim3(64), in, w, g, c, px, nyb);
-    else
-      MLAU_LAUNCH(h, k, (k_sweeps2d<ODR, FLUX, MIX, false>), gr, dim3(64), in, w, g, c, px, nyb);
+    if constexpr (MIX != MLAU_FP64 && !whole_march<FLUX, MIX>) {
+      if (split) {
+        MLAU_LAUNCH(h, k, (k_sweeps2d<ODR, FLUX, MIX, true>), gr, dim3(64), in, w, g, c, px, nyb);
+        return;
+      }
+    }
+    if constexpr (two_waves<ODR, FLUX, MIX>) {
+      if (gr.x > kTwoWaves) {
+        MLAU_LAUNCH(h, k, (k_sweeps2d_two<ODR, FLUX, MIX, false>), gr, dim3(64), in, w, g, c, px, nyb);
+        return;
+      }
+    }
+    MLAU_LAUNCH(h, k, (k_sweeps2d<ODR, FLUX, MIX, false>), gr, dim3(64), in, w, g, c, px, nyb);
   });
 }
 
@@ -251,10 +295,19 @@ static void sweeps2d_inl(Handle *h, const U2 &in, const W2 &w, const G2 &g)
 {
   launch_sweeps2d<MIX>(h, g, ychunk(h, g), K_XSW2D_INL, K_YSW2D_INL,
                        [&](int k, dim3 gr, bool split, int c, unsigned px, unsigned nyb) {
-    if (split)
-      MLAU_LAUNCH(h, k, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, MIX != MLAU_FP64>), gr, dim3(64), in, w, g, c, px, nyb);
-    else
-      MLAU_LAUNCH(h, k, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, false>), gr, dim3(64), in, w, g, c, px, nyb);
+    if constexpr (MIX != MLAU_FP64) {
+      if (split) {
+        MLAU_LAUNCH(h, k, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, true>), gr, dim3(64), in, w, g, c, px, nyb);
+        return;
+      }
+    }
+    if constexpr (two_waves_inl<ODR, FLUX, MIX>) {
+      if (gr.x > kTwoWaves) {
+        MLAU_LAUNCH(h, k, (k_sweeps2d_inl_two<ODR, FLUX, MIX, CTW, false>), gr, dim3(64), in, w, g, c, px, nyb);
+        return;
+      }
+    }
+    MLAU_LAUNCH(h, k, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, false>), gr, dim3(64), in, w, g, c, px, nyb);
   });
 }
 
