@@ -499,23 +499,28 @@ static int win1d_odr(Ensemble *e, EnsGroup *G, int n)
 // per CU by its registers): a window forms 256 cells for the 182 it gives, so
 // a full chip is left to the stages.  Members of 5000 cells, 28 windows each, in
 // FP64 as stages and as windows, us a step: 16 members 42.1 and 30.5, 24 44.0 and
-// 41.0, 32 54.1 and 55.9, 128 156 and 189.  Members that ended are taken to be of
-// the mean size.  Both give the same bits, so a group may change over at any launch.
-static bool windows1d(const Ensemble *e, const EnsGroup *G)
+// 41.0, 32 54.1 and 55.9, 128 156 and 189.  One step by itself takes two launches of windows
+// too, so only while they fill the CUs once: us a call, 256 windows 91 and 86, 352 91 and 104, 700
+// 102 and 120 (two steps 136 and 100, 137 and 129, 160 and 158).  Members that ended are
+// taken to be of the mean size.  Both give the same bits, so a group may change over at any launch.
+static bool windows1d(const Ensemble *e, const EnsGroup *G, int steps)
 {
   if (G->variant != 2) return false;
   long long n = 0;
   for (int id : G->slot_id) n += id >= 0;
-  return G->need[T1_WIN] * G->nrun <= 3ll * ens_cus(e) * n;
+  return G->need[T1_WIN] * G->nrun <= (steps == 1 ? 1ll : 3ll) * ens_cus(e) * n;
 }
 
 // The plan, fill, CFL and dt passes once per 32 steps of windows: 14.7 us a step
 // with 8 of them, 12.8 with 32, 12.7 with 64.
-static int graph_steps1d(const Ensemble *e, const EnsGroup *G) { return windows1d(e, G) ? 4 * e->gsteps : e->gsteps; }
+static int graph_steps1d(const Ensemble *e, const EnsGroup *G)
+{
+  return windows1d(e, G, 4 * e->gsteps) ? 4 * e->gsteps : e->gsteps;
+}
 
 static int launch_many1d(Ensemble *e, EnsGroup *G, int n)
 {
-  if (!windows1d(e, G)) return -1;
+  if (!windows1d(e, G, n)) return -1;
   const int most = graph_steps1d(e, G);
   for (; n > 0; n -= most) {
     const int k = n < most ? n : most;
