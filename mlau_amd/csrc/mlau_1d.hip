@@ -178,20 +178,33 @@ static void step1d(Handle *h)
   }
 }
 
-// Whole steps per launch: more save launches and repeat more cells at the
-// windows' edges.  Measured, us for 32 steps (MUSCL MLAU open / WCNS4 LHLLD periodic), a launch
-// or two per stage -> 1, 2, 4 steps per launch: 1024 cells 843 -> 558, 527, 534 /
-// 1049 -> 673, 625, 597; 65536: 1178 -> 854, 805, 784 / 1704 -> 1247, 1179, 1162;
-// 262144: 2292 -> 2019, 1899, 2193 / 3540 -> 3015, 2884, 3922; 1048576: 6461 -> 6885, 6936,
-// 8170 / 11050 -> 10566, 11347, 14478.  0: separate stage launches, also for the mixed
-// forms, whose multiply-adds the compiler would fuse otherwise here (rounding differences
-// of 1e-16 with FP64 solvers and of 1e-9 to 1e-8 with FP32 or Roe's, between grids on the two sides of
-// the line).
-static int steps_per_launch1d(const Handle *h, bool cfl_mode)
+// Whole steps per launch: 1, 2 or 4.  More save launches (about 1.5 us a step each time) but repeat
+// more cells at the windows' edges, and a step costs as many rounds of the 256 CUs as its windows
+// fill (one window a CU: 11.5 us a round for MUSCL + MLAU, 15.5 for WCNS4 + LHLLD): as many as take no
+// further round.  Measured, us a step with a launch or two per stage and with 1, 2, 4 steps per launch, rk 3
+// (MUSCL + MLAU open / WCNS4 + LHLLD periodic): 20000 cells 24.7 and 13.8, 13.0, 12.4 / 32.8 and 18.9, 17.2, 16.5;
+// 100000 40.2 and 25.1, 23.7, 33.1 / 59.7 and 35.1, 33.3, 47.1; 131072 49.6 and 36.7, 34.2, 33.4 / 70.3 and 51.3, 48.6,
+// 62.4; 300000 72.6 and 60.0, 66.9, 75.5 / 106 and 100, 95.9, 124; 393000 91.3 and 82.4, 78.3, 96.4 /
+// 129 and 117, 128, 155; 1048576 202 and 215, 217, 255 / 345 and 330, 355, 452.
+// 0: separate stage launches.  A periodic grid at ODR 2 takes one launch a stage and is
+// better off so from fewer cells on: 262144 60.1 and 62.0, 58.3, 67.4; 300000 61.9 and 62.5, 69.5; 350000 70.4 and
+// 74.4, 81.1; and for a single step, whose result is copied back, wherever a step takes more than one round:
+// 56000 31.9 and 29.4, 65536 39.3 and 41.9, 200000 62.6 and 71.3.  The mixed forms always: the compiler would
+// fuse their multiply-adds otherwise here (rounding differences of 1e-16 with FP64 solvers and of 1e-9 to
+// 1e-8 with FP32 or Roe's, between grids on the two sides of a line).
+static int steps_per_launch1d(const Handle *h, int nsteps, bool cfl_mode)
 {
+  const int cells = h->g.nx - 8, rk = h->s.rk;
   if ((h->tune & 8) || h->g.nx > 393216 || h->s.precision != MLAU_FP64) return 0;
+  auto rounds = [&](int K) {
+    const int own = kWin1 - 2 * (h->s.odr <= 2 ? win1_halo<2>(K, rk) : win1_halo<4>(K, rk));
+    return ((cells + own - 1) / own + 255) / 256;
+  };
+  if (h->s.odr == 2 && rk >= 2 && h->s.bc1d == MLAU_BC1D_PERIODIC &&
+      (cells > 280000 || (nsteps == 1 && rounds(1) > 1)))
+    return 0;
   if (cfl_mode) return 1;  // the next dt needs the whole grid
-  return h->g.nx > 131072 ? 2 : 4;
+  return rounds(4) <= rounds(1) ? 4 : rounds(2) <= rounds(1) ? 2 : 1;
 }
 
 // Steps in launches of up to `most` whole steps, from one state to the other and
@@ -267,7 +280,7 @@ int run_cfl_1d(Handle *h, double cfl, double vfloor)
 int run_steps_1d(Handle *h, int nsteps, bool cfl_mode, double cfl, double vfloor)
 {
   if (h->g.xoff != 4) return (int)hipErrorInvalidValue;
-  if (const int most = steps_per_launch1d(h, cfl_mode)) {
+  if (const int most = steps_per_launch1d(h, nsteps, cfl_mode)) {
     Steps1Fn fs;
     switch (h->s.odr) {
     case 1: fs = pick1s<1>(h->s.flux); break;
