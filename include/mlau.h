@@ -17,8 +17,9 @@
  *
  * Every call returns MLAU_OK (0) or an error code; mlau_last_error() gives the
  * message of the last failure on the calling thread.  Calls on one handle are
- * serialised on that handle's HIP stream; use a handle from one host thread at
- * a time, distinct handles from distinct threads at once.
+ * serialised on that handle's HIP stream (some large 2D/3D grids run a stage's x sweep
+ * beside the others, on an internal stream that rejoins it within the stage); use a
+ * handle from one host thread at a time, distinct handles from distinct threads at once.
  */
 #ifndef MLAU_H
 #define MLAU_H

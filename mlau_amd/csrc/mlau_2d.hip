@@ -140,6 +140,15 @@ constexpr bool two_waves = (MIX == MLAU_FP64 && ((FLUX == FLUX_MLAU && ODR >= 2)
                            (MIX == MLAU_MIXED_RECON && FLUX == FLUX_MLAU && ODR == 4);
 constexpr unsigned kTwoWaves = 2048;
 
+// The x sweep by itself, four row-flattened wavefronts to a block.
+template <int ODR, int FLUX, int MIX>
+__global__ __launch_bounds__(256) void k_xsweep2d_inl(U2 u, W2 w, G2 g)
+{
+  const long W = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (W >= xsweep_waves(g.ny, g.nx)) return;  // whole wavefront
+  xsweep2d_inl_body<ODR, FLUX, MIX>(u, w, g, W, threadIdx.x & 63);
+}
+
 // CT weight 1/2 at corners 3..nx-3 x 3..ny-3 (no upwind weighting)
 __global__ __launch_bounds__(256) void k_ctx_half2d(W2 w, G2 g)
 {
@@ -293,6 +302,21 @@ static void stage2d(Handle *h, const U2 &in, const U2 &ut, const U2 &out, const 
 template <int ODR, int FLUX, int MIX, int CTW>
 static void sweeps2d_inl(Handle *h, const U2 &in, const W2 &w, const G2 &g)
 {
+  if constexpr (MIX != MLAU_FP64 || ODR == 1) {  // x_beside_2d
+    const int ch = ychunk(h, g);
+    if (!(h->tune & 64) && !split_march<MIX>(ch)) {
+      const unsigned px = (g.nx + 63) / 64, nyb = px * ((g.ny - 5 + ch - 1) / ch);
+      const unsigned xb = (unsigned)((xsweep_waves(g.ny, g.nx) + 3) / 4);
+      if (run_beside(
+              h,
+              [&] { MLAU_LAUNCH(h, K_XSW2D_INL, (k_xsweep2d_inl<ODR, FLUX, MIX>), dim3(xb), dim3(256), in, w, g); },
+              [&] {
+                MLAU_LAUNCH(h, K_YSW2D_INL, (k_sweeps2d_inl<ODR, FLUX, MIX, CTW, false>), dim3(nyb), dim3(64), in, w, g,
+                            ch, px, nyb);
+              }))
+        return;
+    }
+  }
   launch_sweeps2d<MIX>(h, g, ychunk(h, g), K_XSW2D_INL, K_YSW2D_INL,
                        [&](int k, dim3 gr, bool split, int c, unsigned px, unsigned nyb) {
     if constexpr (MIX != MLAU_FP64) {
@@ -372,6 +396,23 @@ static Step2Fn pick2(int flux, int precision)
   case MLAU_MIXED_RECON: return pick2f<ODR, MLAU_MIXED_RECON>(flux);
   default: return pick2f<ODR, MLAU_FP64>(flux);
   }
+}
+
+// Periodic grids whose x sweep, which alone fits three wavefronts a SIMD where the joint launch
+// fits two, runs in a launch of its own beside the y sweep: it pays where the sweeps are light beside
+// their bytes and the grid is large enough to hide the fork and join. us a step, before the sweeps
+// shared a launch, in one launch, beside each other: mixed MUSCL + HLLD 1000^2 393, 408, 403, 1500^2 1005, 1078, 1018,
+// 2048^2 1933, 2087, 1956;
+// mixed_recon 2048^2 2071, 2257, 2152; mixed WCNS4 + LHLLD 1500^2 1342, 1333, 1360, 1750^2 1814, 1843, 1813, 2048^2 2457, 2568,
+// 2485; FP64 ODR 1 + HLLD 1250^2 754, 741, 754, 1500^2 1109, 1140, 1108. mixed_recon + MLAU, whose solver keeps the
+// x sweep to two wavefronts, and the other FP64 forms stay in one launch (WCNS4 + MLAU 2048^2 2826, 2756, 2845).
+bool x_beside_2d(const Handle *h)
+{
+  const int odr = h->s.odr, flux = h->s.flux, mix = h->s.precision;
+  if (!inline2d(h) || (mix == MLAU_FP64 && odr != 1) || (mix != MLAU_MIXED && flux == FLUX_MLAU)) return false;
+  if (mix == MLAU_MIXED && flux == FLUX_HLLD && odr == 2) return h->ncell >= 900000;
+  const bool light = odr <= 2 && (flux == FLUX_HLLD || flux == FLUX_LHLLD);
+  return h->ncell >= (light ? 2100000 : 3000000);
 }
 
 int run_cfl_2d(Handle *h, double cfl, double vfloor)

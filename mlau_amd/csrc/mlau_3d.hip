@@ -90,6 +90,15 @@ __global__ __launch_bounds__(64) MLAU_TWO_WAVES void k_sweeps3d(Sw3 wx, Sw3 wy, 
   }
 }
 
+// The x sweep by itself, four row-flattened wavefronts to a block.
+template <int ODR, int FLUX, int MIX>
+__global__ __launch_bounds__(256) void k_xsweep3d(Sw3 w, G3 g)
+{
+  const long W = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (W >= xsweep_waves((long)g.ny * g.nz, g.nx)) return;  // whole wavefront
+  xsweep3d_body<ODR, FLUX, MIX>(w, g, W, threadIdx.x & 63);
+}
+
 template <int ODR>
 __global__ __launch_bounds__(256) void k_edge3d(Edge3 e, G3 g)
 {
@@ -247,7 +256,14 @@ static void stage3d(Handle *h, const U3 &in, const U3 &ut, const U3 &out, double
     sweeps(K_YSWEEP3D, yb, yb, 0);
     sweeps(K_ZSWEEP3D, zb, 0, zb);
   } else {
-    sweeps(K_SWEEPS3D, yb + zb + (unsigned)xw, yb, zb);
+    bool done = false;
+    if constexpr (MIX != MLAU_FP64 || ODR == 1) {  // x_beside_3d
+      const dim3 xb((unsigned)((xw + 3) / 4));
+      done = !split && run_beside(
+                           h, [&] { MLAU_LAUNCH(h, K_XSWEEP3D, (k_xsweep3d<ODR, FLUX, MIX>), xb, b256, wx, g); },
+                           [&] { sweeps(K_SWEEPS3D, yb + zb, yb, zb); });
+    }
+    if (!done) sweeps(K_SWEEPS3D, yb + zb + (unsigned)xw, yb, zb);
   }
   Edge3 e;
   e.fxt = h->fx[4]; e.fxu = h->fx[5]; e.fcx0 = h->fcx[0]; e.fcx1 = h->fcx[1];
@@ -319,6 +335,17 @@ static Step3Fn pick3(int flux, int precision)
   case MLAU_MIXED_RECON: return pick3f<ODR, MLAU_MIXED_RECON>(flux);
   default: return pick3f<ODR, MLAU_FP64>(flux);
   }
+}
+
+// As x_beside_2d, from 6 million cells on (the y and z sweeps in one launch). us a step, before,
+// in one launch, beside: mixed WCNS4 + LHLLD 150^3 4174, 4107, 4111, 240^3 15113, 15358, 15094; mixed ODR 1 + HLLD 180^3 5485,
+// 5617, 5538, 240^3 12124, 12661, 12440; FP64 ODR 1 + LHLLD 180^3 6226, 6356, 6202; mixed_recon WCNS4 + MLAU 240^3 18855, 18711,
+// 18883 (one launch).
+bool x_beside_3d(const Handle *h)
+{
+  const int mix = h->s.precision;
+  if ((mix == MLAU_FP64 && h->s.odr != 1) || (mix == MLAU_MIXED_RECON && h->s.flux == FLUX_MLAU)) return false;
+  return h->ncell >= 6000000;
 }
 
 int run_cfl_3d(Handle *h, double cfl, double vfloor)

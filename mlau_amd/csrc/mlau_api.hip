@@ -146,6 +146,28 @@ using namespace mlau;
 
 struct mlau_handle : public Handle {};
 
+// The side stream and its events; without them the sweeps run in one launch.
+static void release_side(Handle *h)
+{
+  if (h->side) {
+    hipStreamSynchronize(h->side);
+    hipStreamDestroy(h->side);
+  }
+  if (h->ev_fork) hipEventDestroy(h->ev_fork);
+  if (h->ev_join) hipEventDestroy(h->ev_join);
+  h->side = nullptr;
+  h->ev_fork = h->ev_join = nullptr;
+}
+static void make_side(Handle *h)
+{
+  if (hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking) == hipSuccess &&
+      hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming) == hipSuccess &&
+      hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming) == hipSuccess)
+    return;
+  release_side(h);
+  (void)hipGetLastError();
+}
+
 extern "C" {
 
 const char *mlau_last_error(void) { return g_err.c_str(); }
@@ -194,11 +216,13 @@ int mlau_create(const mlau_grid *grid, const mlau_scheme *scheme, mlau_handle **
     delete h;
     return fail(MLAU_ERR_HIP, "hipStreamCreate failed");
   }
+  if (h->g.dim == 2 ? x_beside_2d(h) : h->g.dim == 3 && x_beside_3d(h)) make_side(h);
   // array budget: 2x state, prims, aux, 3x8 fluxes, 3x2 central parts, 3 edges
   const int nfields = 16 + 8 + 6 + 24 + 6 + 3;
   const size_t per = ((size_t)h->ncell * sizeof(double) + 255) & ~(size_t)255;
   h->base_bytes = per * nfields + 4096;
   if (hipMalloc(&h->base, h->base_bytes) != hipSuccess) {
+    release_side(h);
     hipStreamDestroy(h->stream);
     delete h;
     return fail(MLAU_ERR_NOMEM, "hipMalloc of the resident workspace failed");
@@ -242,6 +266,7 @@ void mlau_destroy(mlau_handle *h)
   for (auto e : h->timing.pool) hipEventDestroy(e);
   if (h->gexec) hipGraphExecDestroy(h->gexec);
   if (h->base) hipFree(h->base);
+  release_side(h);
   if (h->stream) hipStreamDestroy(h->stream);
   delete h;
 }

@@ -77,6 +77,9 @@ struct Handle {
   int nf;                  // 7 (1D) or 8
   long long ncell;         // nx*ny*nz including ghosts
   hipStream_t stream = nullptr;
+  // second stream, where the x sweep runs beside the others (large grids of some forms, else null)
+  hipStream_t side = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   int device = 0;
   double *base = nullptr;  // one device allocation carved into the arrays below
   size_t base_bytes = 0;
@@ -115,6 +118,28 @@ void timing_end(Handle *h, int k, hipEvent_t a);
     hipLaunchKernelGGL(kernel, grid, block, 0, (h)->stream, __VA_ARGS__);             \
     if ((h)->timing.enabled) timing_end((h), (kid), _ev);                             \
   } while (0)
+
+// `beside` on the handle's side stream, between a fork from and a join into its own,
+// and `here` on its own meanwhile; false (nothing launched) where there is no side stream.
+template <typename A, typename B>
+bool run_beside(Handle *h, A here, B beside)
+{
+  const hipStream_t own = h->stream;
+  if (!h->side || hipEventRecord(h->ev_fork, own) != hipSuccess ||
+      hipStreamWaitEvent(h->side, h->ev_fork, 0) != hipSuccess)
+    return false;
+  here();
+  h->stream = h->side;
+  beside();
+  h->stream = own;
+  if (hipEventRecord(h->ev_join, h->side) != hipSuccess || hipStreamWaitEvent(own, h->ev_join, 0) != hipSuccess)
+    hipStreamSynchronize(h->side);
+  return true;
+}
+
+// Whether a handle gets a side stream for its sweeps.
+bool x_beside_2d(const Handle *h);
+bool x_beside_3d(const Handle *h);
 
 // per-dimension drivers (return hipError_t as int)
 int run_steps_1d(Handle *h, int nsteps, bool cfl_mode, double cfl, double vfloor);
