@@ -31,11 +31,9 @@ BYTES_PER_ZONE_UPDATE = 512  # 8 fields x 8 B x 8 passes per full RK3 step
 PROFILE_2048 = {
     "traffic_file": "profiles/vortex2d_2048_fp64_hbm_traffic.md",
     # HBM bytes per launch (update2d: mean of the first-stage and other-stage launches, 1:2)
-    "traffic": {"xsweep2d_inl": 601.4e6, "ysweep2d_inl": 992.9e6, "update2d": (993.2e6 + 2 * 1264.9e6) / 3,
-                "ez2d": 203.8e6, "cfl2d": 285.7e6},
+    "traffic": {"sweeps2d": 1770.8e6, "update2d": (994.3e6 + 2 * 1265.7e6) / 3, "ez2d": 203.8e6, "cfl2d": 286.5e6},
     "fp64_file": "profiles/vortex2d_2048_fp64_valu.md",
-    "fp64": {"xsweep2d_inl": 126.27e6, "ysweep2d_inl": 132.85e6, "update2d": (13.37e6 + 2 * 14.42e6) / 3,
-             "ez2d": 6.11e6, "cfl2d": 4.07e6},
+    "fp64": {"sweeps2d": 259.08e6, "update2d": (13.37e6 + 2 * 14.42e6) / 3, "ez2d": 6.11e6, "cfl2d": 4.07e6},
 }
 
 
