@@ -88,6 +88,11 @@ __device__ __forceinline__ double prim2d_pr(const U2 &u, const G2 &g, const Prim
   return (g.gamma - 1.0) * (u.f[4][s] - 0.5 * (P.ro * P.v2 + b2));
 }
 __device__ __forceinline__ double prim2d_m2(const G2 &g, const Prim2 &P) { return P.v2 / (g.gamma * P.pr * P.iro); }
+// prim2d_m2 >= 1, without its division where that can be.
+__device__ __forceinline__ bool prim2d_ge1(const G2 &g, const Prim2 &P)
+{
+  return ratio_ge1(P.v2, g.gamma * P.pr * P.iro);
+}
 __device__ __forceinline__ int prim2d_sup(const G2 &g, const Prim2 &P)  // ratio_class of prim2d_m2
 {
   return ratio_class(P.v2, g.gamma * P.pr * P.iro);

@@ -124,7 +124,7 @@ __device__ __forceinline__ void ysweep2d_inl_body(const U2 &u, const W2 &w, cons
     W[4][m] = P.bz;
     W[5][m] = P.cx;
     W[6][m] = P.pr;
-    supb = (supb & ~(1u << m)) | ((prim2d_sup(g, P) & 1u) << m);
+    supb = (supb & ~(1u << m)) | ((prim2d_ge1(g, P) ? 1u : 0u) << m);
   };
   // shock sensor dvx of window row m (row R): aux2d_body's expression
   auto dvx = [&](int R, int m) {

@@ -86,7 +86,13 @@ MLAU_DEV int ratio_class(double a, double b)
   }
   return a >= b;
 }
-MLAU_DEV bool ratio_ge1(double a, double b) { return ratio_class(a, b) == 1; }
+// The first class alone, for selectors that do not look at NaN: the class of each row in the
+// marching y sweep cost the mixed joint sweeps 51 more reads of spilled scalars (1300 x 810: 1.5 % of a step).
+MLAU_DEV bool ratio_ge1(double a, double b)
+{
+  if (__builtin_expect(!(b > 0.0 && b < __builtin_huge_val()), 0)) return a / b >= 1.0;
+  return a >= b;
+}
 // dmax(m[0], dmax(m[1], m[2])) >= 1 by the classes of the three: dmax gives its
 // second argument where either is NaN, so the last one's NaN (a cold cell at rest,
 // 0 / 0) decides and the others' do not count.
